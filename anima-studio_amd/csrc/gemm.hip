@@ -2,8 +2,11 @@
 // i8 / w4 B-loaders (gemm.js:129-159), re-designed as W8A8 on the int8 matrix cores.
 //
 //   gemm_i8   C = epi((qx @ qw^T) * s_x[m] * s_w[n]) with v_mfma_i32_32x32x32_i8 (exact int32
-//             accumulation).  Block tile 128x128, k-tile 64, 4 waves of 64x64, double-buffered
-//             LDS with 80-byte rows (conflict-free 16-byte fragment reads).
+//             accumulation): gemm_i8_256 and the smaller tiles of gemm_i8_tile, chosen by size, on
+//             int8 weights (W4: on the unpacked grid); gemm_i8_kernel for unaligned rows, and for W4
+//             weights decoded inside a product that is not given the 256x256 tile: block tile
+//             128x128, k-tile 64, 4 waves of 64x64, double-buffered LDS with 80-byte rows
+//             (conflict-free 16-byte fragment reads).
 //             W4: the weight tile is decoded in the loader, nibble -> int8 grid value through a
 //             16-entry table per 16-weight group.  The table of a group depends only on its fp8
 //             s_rel byte, so each workgroup first builds all 256 possible tables,
@@ -320,23 +323,23 @@ __device__ __forceinline__ void epi_load_c(const GemmArgs& a, int m, int n, f32x
   }
 }
 
-// The plain epilogues with the LoRA B product (gemm_i8_256<..., LORA>), for the wave's 4 x 2
-// tiles of 32 x 32 in the C^T layout, in three phases: (1) every accumulator becomes its fp32
+// The plain epilogues with the LoRA B product (the LORA instances), for the wave's MT x NT (256x256
+// kernel: 4 x 2) tiles of 32 x 32 in the C^T layout, in three phases: (1) every accumulator becomes its fp32
 // y = (acc * s_x) * s_w (* alpha) (+ bias) in place; (2) per 16-k slice of the rank, the slice's
-// operands of all eight tiles are loaded at once -- the B planes of the two column groups (A
+// operands of all tiles are loaded at once -- the B planes of the two column groups (A
 // operand: lane lq holds row n + lq) and the activations of the four row groups (B operand: lane
 // lq holds row m, split into three bf16 terms in registers) -- and six v_mfma_f32_32x32x16_bf16
 // per tile (mfma_s3) add sum_k lx[m][k] * B[n][k] onto y, so that one load latency per slice is
 // exposed, not one per tile; (3) activation and store / residual / gate as in epi_store_t.
 // Every lane takes part in the MFMAs (rows past M and columns past N read zeros).
-template <int BSTEP>
-__device__ __forceinline__ void lora_y(const GemmArgs& a, const i32x16 (&acc)[4][2], int m0, int n0, int hf, int lq,
-                                       const float (&sxv)[4], f32x16 (&y)[4][2]) {
+template <int BSTEP, int MT, int NT>
+__device__ __forceinline__ void lora_y(const GemmArgs& a, const i32x16 (&acc)[MT][NT], int m0, int n0, int hf, int lq,
+                                       const float (&sxv)[MT], f32x16 (&y)[MT][NT]) {
   if (a.acc_out) {  // the raw accumulators first: acc is dead once y is formed
 #pragma unroll
-    for (int j = 0; j < 2; j++)
+    for (int j = 0; j < NT; j++)
 #pragma unroll
-      for (int i = 0; i < 4; i++)
+      for (int i = 0; i < MT; i++)
 #pragma unroll
         for (int q = 0; q < 4; q++) {
           const int m = m0 + 32 * i, nq = n0 + BSTEP * j + 8 * q;
@@ -346,7 +349,7 @@ __device__ __forceinline__ void lora_y(const GemmArgs& a, const i32x16 (&acc)[4]
         }
   }
 #pragma unroll
-  for (int j = 0; j < 2; j++) {
+  for (int j = 0; j < NT; j++) {
     EpiCols c;
     epi_cols(a, n0 + BSTEP * j, c);
 #pragma unroll
@@ -357,7 +360,7 @@ __device__ __forceinline__ void lora_y(const GemmArgs& a, const i32x16 (&acc)[4]
       for (int e = 0; e < 4; e++) {
         const float b = a.bias && ok ? a.bias[nq + e] : 0.0f;
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
+        for (int i = 0; i < MT; i++) {
           float t = (float)acc[i][j][4 * q + e] * sxv[i];
           t = t * c.sw[q][e];
           if (a.alpha != 1.0f) t = t * a.alpha;
@@ -374,10 +377,10 @@ __device__ __forceinline__ void lora_y(const GemmArgs& a, const i32x16 (&acc)[4]
   // vector temporaries from raising the kernel's register pressure into main-loop spills)
   const float* lx = a.lx + (int64_t)__builtin_amdgcn_readfirstlane(a.lcols ? (n0 / a.lcols) * a.lr : 0);
   for (int k0 = 0; k0 < a.lr; k0 += 16) {
-    bf16x8 bv[2][3];
-    float4 xr[4][2];
+    bf16x8 bv[NT][3];
+    float4 xr[MT][2];
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
+    for (int j = 0; j < NT; j++) {
       const int nr = n0 - 4 * hf + BSTEP * j + lq;
       const bool nok = nr < a.N;
       const uint16_t* bp = a.lb + (int64_t)(nok ? nr : 0) * a.lr + 8 * hf + k0;
@@ -385,7 +388,7 @@ __device__ __forceinline__ void lora_y(const GemmArgs& a, const i32x16 (&acc)[4]
       for (int p = 0; p < 3; p++) bv[j][p] = nok ? ld_bf8(bp + p * plane) : z8;
     }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < MT; i++) {
       const int m = m0 + 32 * i;
       const bool mok = m < a.M;
       const float* xp = lx + (int64_t)(mok ? m : 0) * a.ld_lx + 8 * hf + k0;
@@ -393,22 +396,22 @@ __device__ __forceinline__ void lora_y(const GemmArgs& a, const i32x16 (&acc)[4]
       xr[i][1] = mok ? *(const float4*)(xp + 4) : z4;
     }
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < MT; i++) {
       bf16x8 xv[3];
       split3(xr[i][0], xr[i][1], xv);
 #pragma unroll
-      for (int j = 0; j < 2; j++) y[i][j] = mfma_s3(bv[j], xv, y[i][j]);
+      for (int j = 0; j < NT; j++) y[i][j] = mfma_s3(bv[j], xv, y[i][j]);
     }
   }
 }
 
 // Phase (3) of the LoRA epilogue: activation and store / residual / gate of y.
-template <int EPI, int BSTEP>
-__device__ __forceinline__ void lora_store(const GemmArgs& a, const f32x16 (&y)[4][2], int m0, int n0) {
+template <int EPI, int BSTEP, int MT, int NT>
+__device__ __forceinline__ void lora_store(const GemmArgs& a, const f32x16 (&y)[MT][NT], int m0, int n0) {
 #pragma unroll
-  for (int j = 0; j < 2; j++)
+  for (int j = 0; j < NT; j++)
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
+    for (int i = 0; i < MT; i++) {
       // one tile at a time: keeps the residual loads from being hoisted above the earlier tiles'
       // stores (32 residual quads in flight would not fit beside the 128 registers of y)
       __builtin_amdgcn_sched_barrier(0);
@@ -445,10 +448,10 @@ __device__ __forceinline__ void lora_store(const GemmArgs& a, const f32x16 (&y)[
     }
 }
 
-template <int EPI>
-__device__ __forceinline__ void lora_epilogue(const GemmArgs& a, const i32x16 (&acc)[4][2], int m0, int n0, int hf,
-                                              int lq, const float (&sxv)[4]) {
-  f32x16 y[4][2];
+template <int EPI, int MT, int NT>
+__device__ __forceinline__ void lora_epilogue(const GemmArgs& a, const i32x16 (&acc)[MT][NT], int m0, int n0, int hf,
+                                              int lq, const float (&sxv)[MT]) {
+  f32x16 y[MT][NT];
   lora_y<32>(a, acc, m0, n0, hf, lq, sxv, y);
   lora_store<EPI, 32>(a, y, m0, n0);
 }
@@ -532,12 +535,12 @@ __device__ __forceinline__ f32x4 kv_epi_y(const GemmArgs& a, const i32x16& v, in
 // Q (the prepared-Q form of the attention) goes through the same steps: its own weights (none:
 // no RMSNorm), RoPE when a.qrope, then times a.qc (the attention's scale * log2(e)) before the
 // bf16 rounding, into row-major [M][H][128].
-template <bool Q, class YF>
-__device__ __forceinline__ void kv_epi_k(const GemmArgs& a, const YF& yf, int m0, int n0, int col0, int wave, int hf,
-                                         int lq, float* xch) {
-  const int grp = (wave >> 1) & 1;
+// MT: row groups of the wave; grp: which 32 of the head's first 64 columns (and of its last 64) the
+// wave holds; own / other: the wave's and its partner's 32 MT floats of exchange space.
+template <bool Q, int MT, class YF>
+__device__ __forceinline__ void kv_epi_k(const GemmArgs& a, const YF& yf, int m0, int head, int grp, int hf, int lq,
+                                         float* own, const float* partner) {
   const int c0 = 32 * grp + 4 * hf;  // this lane's first column within the head (< 64)
-  const int head = (col0 - (Q ? 0 : a.kcol)) / HD_K + (wave >> 2);
   const float* wn = Q ? a.qn : a.kn;
   const bool norm = !Q || wn, rope = !Q || a.qrope;  // (uniform over the workgroup)
   // One 32-row block at a time: the partial sum of squares over this lane pair's 64 columns goes
@@ -545,7 +548,7 @@ __device__ __forceinline__ void kv_epi_k(const GemmArgs& a, const YF& yf, int m0
   // recomputed (the same fp32 bits), normalized, rotated, rounded and stored.  (One barrier for all
   // four blocks keeps the first pass's values alive into the second: the spills cost more.)
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
+  for (int i = 0; i < MT; i++) {
     float rn = 1.0f;
     if (norm) {
       float lf[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -559,12 +562,12 @@ __device__ __forceinline__ void kv_epi_k(const GemmArgs& a, const YF& yf, int m0
         }
       float part = (lf[0] + lf[1]) + (lf[2] + lf[3]);
       part = part + __shfl_xor(part, 32);
-      if (hf == 0) xch[wave * 128 + 32 * i + lq] = part;
+      if (hf == 0) own[32 * i + lq] = part;
       __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): the partial sums are in LDS
       asm volatile("" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      const float other = xch[(wave ^ 2) * 128 + 32 * i + lq];
+      const float other = partner[32 * i + lq];
       const float ss = grp == 0 ? part + other : other + part;
       rn = 1.0f / sqrtf(__builtin_fmaf(ss, 1.0f / 128.0f, a.eps));
     }
@@ -615,15 +618,13 @@ __device__ __forceinline__ void kv_epi_k(const GemmArgs& a, const YF& yf, int m0
 // each pair of lanes lq, lq ^ 1 (tokens 2t, 2t + 1: adjacent in the key order too) trades
 // columns and stores 4-byte token pairs, the even lane those of columns e = 0, 1, the odd lane
 // e = 2, 3.  Key order of V^T within each 16-key group: keys 0-3, 8-11, 4-7, 12-15.
-template <class YF>
-__device__ __forceinline__ void kv_epi_v(const GemmArgs& a, const YF& yf, int m0, int n0, int col0, int wave, int hf,
-                                         int lq) {
-  const int c0 = 32 * ((wave >> 1) & 1) + 4 * hf;
-  const int head = (col0 - a.vcol) / HD_K + (wave >> 2);
+template <int MT, class YF>
+__device__ __forceinline__ void kv_epi_v(const GemmArgs& a, const YF& yf, int m0, int head, int grp, int hf, int lq) {
+  const int c0 = 32 * grp + 4 * hf;
   const bool odd = lq & 1;
   bf16* vt = (bf16*)((char*)a.kv + a.kv_plane);
 #pragma unroll
-  for (int i = 0; i < 4; i++) {
+  for (int i = 0; i < MT; i++) {
     const int m = m0 + 32 * i;
     const int mp = m - (odd ? 1 : 0);  // the pair's even token
     const int b = mp / a.L, l = mp - b * a.L;
@@ -1005,6 +1006,9 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_256(GemmArgs a) {
       int tm, tn;
       tile_mn(first + k * stride, tm, tn);
       const int col0 = tn * 256, m0 = tm * 256 + wm + lq, n0 = col0 + bc0 + 4 * hf;
+      const int grp = (wave >> 1) & 1, kh = (col0 - a.kcol) / HD_K + (wave >> 2);
+      float* const xch = (float*)(smem + G2_NST * G2_ST + (W4 ? 4096 : 0));
+      float *const own = xch + 128 * wave, *const other = xch + 128 * (wave ^ 2);
       float sxv[4];
 #pragma unroll
       for (int i = 0; i < 4; i++) sxv[i] = m0 + 32 * i < a.M ? a.sx[m0 + 32 * i] : 0.0f;
@@ -1016,16 +1020,14 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_256(GemmArgs a) {
         const auto yf = [&](int i, int j, int q) {
           return f32x4{y[i][j][4 * q], y[i][j][4 * q + 1], y[i][j][4 * q + 2], y[i][j][4 * q + 3]};
         };
-        float* xch = (float*)(smem + G2_NST * G2_ST + (W4 ? 4096 : 0));
-        if (QP && col0 < a.kcol) kv_epi_k<true>(a, yf, m0, n0, col0, wave, hf, lq, xch);
+        if (QP && col0 < a.kcol) kv_epi_k<true, 4>(a, yf, m0, col0 / HD_K + (wave >> 2), grp, hf, lq, own, other);
         else if (col0 < a.kcol) lora_store<ANIMA_EPI_STORE, 64>(a, y, m0, n0);
-        else if (col0 < a.vcol) kv_epi_k<false>(a, yf, m0, n0, col0, wave, hf, lq, xch);
-        else kv_epi_v(a, yf, m0, n0, col0, wave, hf, lq);
+        else if (col0 < a.vcol) kv_epi_k<false, 4>(a, yf, m0, kh, grp, hf, lq, own, other);
+        else kv_epi_v<4>(a, yf, m0, (col0 - a.vcol) / HD_K + (wave >> 2), grp, hf, lq);
       } else {
         const auto yf = [&](int i, int j, int q) { return kv_epi_y(a, acc[i][j], q, sxv[i], n0 + 64 * j); };
-        float* xch = (float*)(smem + G2_NST * G2_ST + (W4 ? 4096 : 0));
         if (QP && col0 < a.kcol) {
-          kv_epi_k<true>(a, yf, m0, n0, col0, wave, hf, lq, xch);
+          kv_epi_k<true, 4>(a, yf, m0, col0 / HD_K + (wave >> 2), grp, hf, lq, own, other);
         } else if (col0 < a.kcol) {
           EpiCols cc;
           const f32x4 none[4] = {};
@@ -1036,9 +1038,9 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_256(GemmArgs a) {
             for (int i = 0; i < 4; i++) epi_store_t<ANIMA_EPI_STORE>(a, acc[i][j], m0 + 32 * i, n0 + 64 * j, sxv[i], cc, none);
           }
         } else if (col0 < a.vcol) {
-          kv_epi_k<false>(a, yf, m0, n0, col0, wave, hf, lq, xch);
+          kv_epi_k<false, 4>(a, yf, m0, kh, grp, hf, lq, own, other);
         } else {
-          kv_epi_v(a, yf, m0, n0, col0, wave, hf, lq);
+          kv_epi_v<4>(a, yf, m0, (col0 - a.vcol) / HD_K + (wave >> 2), grp, hf, lq);
         }
       }
 #pragma unroll
@@ -1100,6 +1102,212 @@ __global__ __launch_bounds__(512, 1) void gemm_i8_256(GemmArgs a) {
     if (g + 1 < total) iteration(g + 1, std::integral_constant<int, 1>{});
   }
   G2_WAIT_VM(0);  // no copy into LDS outlives the workgroup
+}
+// ------------------------------------------------------------------ int8 kernel for smaller grids
+//
+// gemm_i8_tile: one BM x BN output tile per workgroup, waves of WM x WN with the weight fragment as
+// srcA (the C^T layout and epilogues of the 256x256 kernel).  A stage holds 128 k bytes of the
+// tile's rows (whole cache lines per row); KG k-groups of waves take 4 / KG of its four 32-byte
+// k-steps each, and the groups' int32 sums are added through LDS at the end (exact: the result
+// depends neither on the tile nor on the split).  NST LDS stages, filled NST - 1 ahead by
+// buffer_load_dwordx4 ... lds, one barrier per stage.  LDS row r holds eight 16-byte k units, unit u
+// at slot u ^ (r % 8), so eight consecutive rows' reads of one unit touch every bank once.  Rows
+// past M (N) lie past the buffer resource's end and read as zero: the row part of every copy's
+// address is in the vector offset, so the scalar offset (the k position) never passes the
+// resource's size.
+// one 1 KiB copy (a wave's 64 lanes x 16 bytes) into LDS
+__device__ __forceinline__ void gt_copy(__amdgpu_buffer_rsrc_t r, char* dst, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void_t*)dst, 16, voff, soff, 0, 0);
+}
+
+template <int BM, int BN, int WM, int WN, int SK, int KG, int NST, int MINW, int EPI, bool KV, bool QP, bool LORA>
+__global__ __launch_bounds__(64 * (BM / WM) * (BN / WN) * KG, MINW) void gemm_i8_tile(GemmArgs a) {
+  constexpr int NWM = BM / WM, NWN = BN / WN, NWT = NWM * NWN, NW = NWT * KG;  // waves
+  constexpr int MT = WM / 32, NT = WN / 32;
+  constexpr int ST = (BM + BN) * SK, KS = SK / 32 / KG;     // bytes of a stage; k-steps per group
+  constexpr int UN = SK / 16, CR = 64 / UN;                 // 16-byte units of a row; rows of a 1 KiB copy
+  constexpr int CPW = ST / 1024 / NW;                       // 1 KiB copies per wave and stage
+  static_assert(CPW * NW * 1024 == ST, "whole copies per wave");
+  static_assert(!KV || (BN == 128 && WN == 64 && KG == 1 && EPI == ANIMA_EPI_STORE), "one head per tile");
+  static_assert(NST >= 3, "a stage being read, one published, one in flight");
+  static_assert((KG == 1 || KG == 2) && NWT * 64 * MT * NT * 64 * (KG - 1) <= NST * ST, "the k-groups' sums fit the stages");
+  __shared__ __attribute__((aligned(1024))) char smem[NST * ST + (KV ? NW * 32 * MT * 4 : 0)];
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+  const int lq = lane & 31, hf = lane >> 5;
+  const int ntn = (a.N + BN - 1) / BN, ntm = (a.M + BM - 1) / BM;
+  int tm, tn;
+  {
+    // XCD x takes a contiguous range of tiles (dispatch is round-robin over the 8 XCDs), in groups
+    // of 8 row tiles, column-major inside a group: the tiles in flight on one XCD share rows of A
+    // and of B in its L2
+    const int total = ntn * ntm, q = total >> 3, r = total & 7, x = blockIdx.x & 7;
+    const int t = x * q + min(x, r) + (int)(blockIdx.x >> 3);
+    const int grp = t / (8 * ntn), row0 = 8 * grp, gm = min(8, ntm - row0), local = t - grp * 8 * ntn;
+    tn = local / gm;
+    tm = row0 + (local - tn * gm);
+  }
+  const int bm = tm * BM, bn = tn * BN, K = a.K;
+  const int kg = wave / NWT, wt = wave % NWT;
+  const int wm = (wt % NWM) * WM, wn = (wt / NWM) * WN;
+  // KV: the wave's two column groups are 64 apart (the RoPE pairs of a head)
+  const int bc0 = KV ? 32 * (wt / NWM) : wn;
+  constexpr int BSTEP = KV ? 64 : 32;
+  const int nk = (K + SK - 1) / SK;  // stages
+
+  __amdgpu_buffer_rsrc_t ra =
+      __builtin_amdgcn_make_buffer_rsrc((void*)(a.qx + (int64_t)bm * K), (short)0, min(BM, a.M - bm) * K, 0x00020000);
+  __amdgpu_buffer_rsrc_t rb = __builtin_amdgcn_make_buffer_rsrc((void*)((const int8_t*)a.w + (int64_t)bn * K), (short)0,
+                                                                min(BN, a.N - bn) * K, 0x00020000);
+  // copy c of this wave: CR rows (A rows first) of SK bytes; lane -> row lane / UN, slot lane % UN
+  const int swz = SK == 128 ? (lane >> 3) & 7 : (lane >> 4) & 3;  // of rows lane / UN + a multiple of CR
+  const int unit = (lane % UN) ^ swz;
+  int voff[CPW];
+  bool isb[CPW];
+#pragma unroll
+  for (int c = 0; c < CPW; c++) {
+    const int ch = wave * CPW + c;
+    isb[c] = ch >= BM / CR;
+    voff[c] = (CR * (isb[c] ? ch - BM / CR : ch) + lane / UN) * K + 16 * unit;
+  }
+  // SK = 128: the last stage of a row with K % 128 == 64 has no second half: those lanes read past
+  // the resource's end (zeros), so the extra k-steps add nothing
+  const int past = unit >= 4 ? 1 << 30 : 0;
+  int icur = 0, ik = 0;  // next stage to fill: its buffer and its first k byte
+  auto issue = [&]() {
+    char* st = smem + icur * ST + wave * CPW * 1024;
+    icur = icur + 1 == NST ? 0 : icur + 1;
+    const int vx = SK == 128 && ik + 64 == K ? past : 0;
+#pragma unroll
+    for (int c = 0; c < CPW; c++) gt_copy(isb[c] ? rb : ra, st + c * 1024, voff[c] + vx, min(ik, K - 64));
+    ik += SK;
+  };
+  int fofs[KS];
+#pragma unroll
+  for (int ks = 0; ks < KS; ks++) fofs[ks] = lq * SK + 16 * ((2 * (kg * KS + ks) + hf) ^ (SK == 128 ? lq & 7 : (lq >> 2) & 3));
+
+  i32x16 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; i++)
+#pragma unroll
+    for (int j = 0; j < NT; j++) acc[i][j] = (i32x16){};
+
+  // k-step ks of a stage from `st` into fragment set p; read r of MT + NT, B first
+  i32x4 af[2][MT], bf[2][NT];
+  auto rd = [&](int p, const char* st, int ks, int r) __attribute__((always_inline)) {
+    if (r < NT) bf[p][r] = *(const i32x4*)(st + (BM + bc0 + BSTEP * r) * SK + fofs[ks]);
+    else af[p][r - NT] = *(const i32x4*)(st + (wm + 32 * (r - NT)) * SK + fofs[ks]);
+  };
+#pragma unroll
+  for (int g = 0; g < NST - 1; g++) issue();  // (past the last stage: re-reads of the last bytes)
+  G2_WAIT_VM(CPW * (NST - 2));
+  g2_barrier();
+#pragma unroll
+  for (int r = 0; r < MT + NT; r++) rd(0, smem, 0, r);
+  int cur = 0;
+  for (int g = 0; g < nk; g++) {
+    // stage g + 1 is published one iteration before its products: its copies are done once at most
+    // those of the NST - 3 stages after it pend; the barrier also ends every wave's reads of stage
+    // g - 1, whose buffer is refilled
+    G2_WAIT_VM(CPW * (NST - 3));
+    g2_barrier();
+    issue();
+    const char* st = smem + cur * ST;
+    cur = cur + 1 == NST ? 0 : cur + 1;
+    const char* sn = smem + cur * ST;
+    // each MFMA is followed by its share of the next k-step's fragment reads (the last k-step reads
+    // stage g + 1, after the last stage a stale one whose values are unused)
+#pragma unroll
+    for (int ks = 0; ks < KS; ks++) {
+      const int p = ks & 1;
+#pragma unroll
+      for (int q = 0; q < MT * NT; q++) {
+        acc[q / NT][q % NT] = __builtin_amdgcn_mfma_i32_32x32x32_i8(bf[p][q % NT], af[p][q / NT], acc[q / NT][q % NT], 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < MT + NT; r++)
+          if (r * MT * NT / (MT + NT) == q) rd(p ^ 1, ks + 1 < KS ? st : sn, ks + 1 < KS ? ks + 1 : 0, r);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  G2_WAIT_VM(0);  // no copy into LDS outlives the loop
+
+  if constexpr (KG > 1) {
+    __syncthreads();
+    i32x4* part = (i32x4*)smem;  // [kg - 1][tile, quad][thread of the group]
+    const int t = wt * 64 + lane;
+    if (kg > 0) {
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+          for (int q = 0; q < 4; q++)
+            part[(((kg - 1) * MT * NT + i * NT + j) * 4 + q) * (NWT * 64) + t] =
+                i32x4{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
+    }
+    __syncthreads();
+    if (kg > 0) return;
+#pragma unroll
+    for (int o = 0; o < KG - 1; o++)
+#pragma unroll
+      for (int i = 0; i < MT; i++)
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const i32x4 v = part[((o * MT * NT + i * NT + j) * 4 + q) * (NWT * 64) + t];
+#pragma unroll
+            for (int e = 0; e < 4; e++) acc[i][j][4 * q + e] += v[e];
+          }
+  }
+
+  const int m0 = bm + wm + lq, n0 = bn + bc0 + 4 * hf;
+  float sxv[MT];
+#pragma unroll
+  for (int i = 0; i < MT; i++) sxv[i] = m0 + 32 * i < a.M ? a.sx[m0 + 32 * i] : 0.0f;
+  if constexpr (KV) {
+    const int grp = wt / NWM;
+    float* const xch = (float*)(smem + NST * ST);
+    float *const own = xch + 32 * MT * wave, *const other = xch + 32 * MT * (wave ^ NWM);
+    // false: Q columns that leave as fp32 rows, by the plain store below
+    const auto operands = [&](const auto& yf) __attribute__((always_inline)) {
+      if (QP && bn < a.kcol) kv_epi_k<true, MT>(a, yf, m0, bn / HD_K, grp, hf, lq, own, other);
+      else if (bn < a.kcol) return false;
+      else if (bn < a.vcol) kv_epi_k<false, MT>(a, yf, m0, (bn - a.kcol) / HD_K, grp, hf, lq, own, other);
+      else kv_epi_v<MT>(a, yf, m0, (bn - a.vcol) / HD_K, grp, hf, lq);
+      return true;
+    };
+    if constexpr (LORA) {
+      f32x16 y[MT][NT];
+      lora_y<BSTEP>(a, acc, m0, n0, hf, lq, sxv, y);
+      if (!operands([&](int i, int j, int q) {
+            return f32x4{y[i][j][4 * q], y[i][j][4 * q + 1], y[i][j][4 * q + 2], y[i][j][4 * q + 3]};
+          }))
+        lora_store<EPI, BSTEP>(a, y, m0, n0);
+      return;
+    } else {
+      if (operands([&](int i, int j, int q) { return kv_epi_y(a, acc[i][j], q, sxv[i], n0 + 64 * j); })) return;
+    }
+  }
+  if constexpr (LORA) {
+    lora_epilogue<EPI>(a, acc, m0, n0, hf, lq, sxv);
+    return;
+  }
+  // one 32 x 32 tile at a time, the next tile's residual loads issued before the current stores
+  f32x4 cv[2][4];
+  EpiCols cc;
+  if constexpr (EPI != ANIMA_EPI_STORE) epi_load_c(a, m0, n0, cv[0]);
+#pragma unroll
+  for (int j = 0; j < NT; j++) {
+    epi_cols(a, n0 + BSTEP * j, cc);
+#pragma unroll
+    for (int i = 0; i < MT; i++) {
+      const int t = j * MT + i;
+      if constexpr (EPI != ANIMA_EPI_STORE)
+        if (t + 1 < MT * NT) epi_load_c(a, m0 + 32 * ((t + 1) % MT), n0 + BSTEP * ((t + 1) / MT), cv[(t + 1) & 1]);
+      epi_store_t<EPI>(a, acc[i][j], m0 + 32 * i, n0 + BSTEP * j, sxv[i], cc, cv[t & 1]);
+    }
+  }
 }
 #undef G2_WAIT_VM
 #undef G2_ISSUE
@@ -2221,6 +2429,78 @@ __global__ __launch_bounds__(256) void gemv_f32w_kernel(F32WArgs a) {
 
 static bool al(const void* p, int b) { return ((uintptr_t)p & (b - 1)) == 0; }
 
+// The int8 kernels by tile: what runs on fewer tiles than CUs is bound by the depth of its k loop,
+// so small products take small tiles (more of them), and products of several rounds take the tile
+// whose last round is fullest.
+enum { GT_256, GT_256x128, GT_128, GT_64x128, GT_32x64, GT_COUNT };
+enum { GT_PLAIN, GT_LORA, GT_OPERANDS, GT_OPERANDS_LORA };  // epilogues
+
+static int gemm_i8_cols(int tile) { return tile == GT_256 ? 256 : tile == GT_32x64 ? 64 : 128; }
+
+// Measured time of one output tile per CU, microseconds: base (launch, first loads, epilogue) +
+// step * K / 2048, for each further tile per CU step * K / 2048 more.  Fitted to M = 256 .. 8192,
+// N = 2048 / 6144 / 8192, K = 2048 / 8192, at K = 2048 and M x N of 256 x 2048: 32x64 6.8 (128x128
+// 16); 1024 x 2048: 64x128 12.4 (256x256 39.5, the former 128x128 loop 38.6; K = 8192 29.8 / 97 /
+// 104); 2240 x 2048: 256x128 27.7 (43.7); 2240 x 8192: 128x128 63 (69.6); 7904 x 2048: 256x256 57.4
+// (128x128 66.7).
+static int gemm_i8_choose(anima_ctx* c, int64_t M, int N, int K, int kind) {
+  static const struct { int bm, bn; float base, step; } T[GT_COUNT] = {
+      {256, 256, 18.0f, 24.0f}, {256, 128, 8.0f, 17.0f}, {128, 128, 8.5f, 9.0f}, {64, 128, 6.0f, 6.5f}, {32, 64, 3.3f, 3.5f}};
+  int best = -1;
+  float bt = 0.0f;
+  for (int t = 0; t < GT_COUNT; t++) {
+    if (t == GT_32x64 && kind != GT_PLAIN) continue;  // (a head, or a rank block, is 128 columns wide)
+    const int64_t tiles = (N + T[t].bn - 1) / T[t].bn * ((M + T[t].bm - 1) / T[t].bm);
+    if (tiles > 0x7fffffff || (t != GT_256 && K > 65536)) continue;  // (tile rows times K: 32-bit offsets)
+    const float us = T[t].base + T[t].step * (float)K / 2048.0f * (float)((tiles + c->num_cus - 1) / c->num_cus);
+    if (best < 0 || us < bt) {
+      best = t;
+      bt = us;
+    }
+  }
+  return best;
+}
+
+template <int EPI, bool KV, bool QP, bool LORA>
+static void gemm_i8_launch_t(anima_ctx* c, const GemmArgs& g, int tile, bool w4) {
+  const auto tiles = [&](int bm, int bn) { return (unsigned)((int64_t)((g.N + bn - 1) / bn) * ((g.M + bm - 1) / bm)); };
+  if (tile == GT_256) {  // persistent: one workgroup per CU at most
+    const unsigned n = tiles(256, 256);
+    const dim3 grid(n < (unsigned)c->num_cus && KV ? n : (unsigned)c->num_cus), block(512);
+    if constexpr (!LORA) {
+      if (w4) {
+        hipLaunchKernelGGL((gemm_i8_256<EPI, true, KV, false, QP>), grid, block, 0, c->stream, g);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((gemm_i8_256<EPI, false, KV, LORA, QP>), grid, block, 0, c->stream, g);
+  } else if (tile == GT_256x128) {
+    hipLaunchKernelGGL((gemm_i8_tile<256, 128, 64, 64, 128, 1, 3, 2, EPI, KV, QP, LORA>), dim3(tiles(256, 128)), dim3(512), 0, c->stream, g);
+  } else if (tile == GT_128) {
+    hipLaunchKernelGGL((gemm_i8_tile<128, 128, 64, 64, 64, 1, 4, 2, EPI, KV, QP, LORA>), dim3(tiles(128, 128)), dim3(256), 0, c->stream, g);
+  } else if (tile == GT_64x128) {
+    if constexpr (KV)
+      hipLaunchKernelGGL((gemm_i8_tile<64, 128, 32, 64, 64, 1, 4, 2, EPI, KV, QP, LORA>), dim3(tiles(64, 128)), dim3(256), 0, c->stream, g);
+    else
+      hipLaunchKernelGGL((gemm_i8_tile<64, 128, 64, 32, 128, 2, 4, 2, EPI, KV, QP, LORA>), dim3(tiles(64, 128)), dim3(512), 0, c->stream, g);
+  } else if constexpr (!KV && !LORA) {
+    hipLaunchKernelGGL((gemm_i8_tile<32, 64, 32, 32, 128, 2, 4, 3, EPI, KV, QP, LORA>), dim3(tiles(32, 64)), dim3(256), 0, c->stream, g);
+  }
+}
+
+// A product with g's epilogue (g.lr: with the LoRA term in it).
+static void gemm_i8_launch(anima_ctx* c, const GemmArgs& g, int tile, bool w4) {
+#define GT_EPI(E)                                                            \
+  {                                                                          \
+    if (g.lr) gemm_i8_launch_t<E, false, false, true>(c, g, tile, w4);       \
+    else gemm_i8_launch_t<E, false, false, false>(c, g, tile, w4);           \
+  }
+  if (g.epi == ANIMA_EPI_STORE) GT_EPI(ANIMA_EPI_STORE)
+  else if (g.epi == ANIMA_EPI_RESID) GT_EPI(ANIMA_EPI_RESID)
+  else GT_EPI(ANIMA_EPI_GATED)
+#undef GT_EPI
+}
+
 int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
   const anima_weight* W = d->W;
   if (!W) return fail(c, ANIMA_E_ARG, "anima_linear: null weight");
@@ -2461,29 +2741,31 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
     g.lcols = d->lora_cols;
   }
   int rc = ANIMA_OK;
-  // Grids that give every CU a 256x256 tile run the persistent 256 kernel, smaller grids the
-  // 128x128 kernel; both unpack W4 codes inside the GEMM.
-  // The 256 kernel's epilogue moves 16-byte column groups: it needs N % 4 == 0 and 16-byte
-  // aligned output rows, scales, bias and gate.
-  const int64_t tiles256 = (int64_t)((N + 255) / 256) * ((M + 255) / 256);
+  // The tiled kernels' epilogues move 16-byte column groups: they need N % 4 == 0 and 16-byte
+  // aligned output rows, scales, bias and gate (gemm_i8_kernel takes what is left).
   const bool vec = N % 4 == 0 && g.ldc % 4 == 0 && al(g.out, 16) && al(g.sw, 16) && (!g.bias || al(g.bias, 16)) &&
                    (g.epi != ANIMA_EPI_GATED || al(g.gate + g.gate_off, 16)) && (!g.add || (al(g.add, 16) && g.ld_add % 4 == 0));
-  const bool big = vec && tiles256 >= c->num_cus && tiles256 <= 0x7fffffff;
+  int tile = vec ? gemm_i8_choose(c, M, N, K, lora ? GT_LORA : GT_PLAIN) : -1;
+  // the LoRA product in the epilogue: a tile's columns lie in one rank block
+  const bool lepi = lora && tile >= 0 && d->lora_cols % gemm_i8_cols(tile) == 0;
   void* grid8 = nullptr;
   bool w4k = w4;  // the GEMM unpacks W4 codes itself
   // (a LoRA epilogue always runs on the int8 grid: the in-GEMM unpack leaves it no registers)
-  if (big && w4 && (c->w4_path == ANIMA_W4_GRID_SCRATCH || lora)) {
+  if (w4 && tile >= 0 && (c->w4_path == ANIMA_W4_GRID_SCRATCH || (tile == GT_256 && lora))) {
     rc = w4_grid_scratch(c, W, g, &grid8);
-    if (rc) {
+    // no memory for the grid: only the 256x256 kernel's callers ever depended on it
+    if (rc && !(rc == ANIMA_E_OOM && tile != GT_256)) {
       if (tmp) anima_free(c, tmp);
       return rc;
     }
-    w4k = false;
+    if (!rc) w4k = false;
+    rc = ANIMA_OK;
   }
-  // small grids, and rank blocks that split a 256-column tile: the LoRA product as an add term
-  // (the split-bf16 kernel, one product per rank block over its columns' rows of the B planes)
+  if (w4k && tile != GT_256) tile = -1;
+  // otherwise the LoRA product is an add term (the split-bf16 kernel, one product per rank block
+  // over its columns' rows of the B planes)
   void* ldelta = nullptr;
-  if (lora && (!big || d->lora_cols % 256)) {
+  if (lora && !(lepi && tile >= 0)) {
     rc = anima_alloc(c, (size_t)M * N * 4, &ldelta);
     if (rc) {
       if (grid8) anima_free(c, grid8);
@@ -2509,24 +2791,8 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
   }
   if (!rc) {
     Launch L(c, w4k ? "gemm.w4a8" : "gemm.i8", 2.0 * M * N * K, 0.0);
-    if (big) {
-      const dim3 grid((unsigned)c->num_cus), block(512);
-#define G2L(E, W)                                                                                    \
-  {                                                                                                  \
-    if (lora) hipLaunchKernelGGL((gemm_i8_256<E, false, false, true>), grid, block, 0, c->stream, g); \
-    else hipLaunchKernelGGL((gemm_i8_256<E, W>), grid, block, 0, c->stream, g);                       \
-  }
-      if (g.epi == ANIMA_EPI_STORE) {
-        if (w4k) G2L(ANIMA_EPI_STORE, true)
-        else G2L(ANIMA_EPI_STORE, false)
-      } else if (g.epi == ANIMA_EPI_RESID) {
-        if (w4k) G2L(ANIMA_EPI_RESID, true)
-        else G2L(ANIMA_EPI_RESID, false)
-      } else {
-        if (w4k) G2L(ANIMA_EPI_GATED, true)
-        else G2L(ANIMA_EPI_GATED, false)
-      }
-#undef G2L
+    if (tile >= 0) {
+      gemm_i8_launch(c, g, tile, w4k);
     } else {
       dim3 grid((N + GBN - 1) / GBN, (unsigned)((M + GBM - 1) / GBM));
       if (w4) hipLaunchKernelGGL(gemm_i8_kernel<true>, grid, dim3(256), 0, c->stream, g);
@@ -2651,17 +2917,14 @@ int linear_qkv_launch(anima_ctx* c, const anima_linear_desc* d, const anima_qkv_
   }
   {
     Launch L(c, w4 ? "gemm.w4a8_qkv" : "gemm.i8_qkv", 2.0 * M * N * K, 0.0);
-    // persistent 256 x 256 tiles (a tile holds two whole heads); one workgroup per CU at most
-    const int64_t tiles = (int64_t)(N / 256) * ((M + 255) / 256);
-    const dim3 grid((unsigned)(tiles < c->num_cus ? tiles : c->num_cus)), block(512);
+    // (a 256-column tile holds two whole heads, a 128-column tile one; in-GEMM W4 decode: 256x256 only)
+    const int tile = w4 ? (int)GT_256 : gemm_i8_choose(c, M, N, K, lora ? GT_OPERANDS_LORA : GT_OPERANDS);
     // (the prepared-Q epilogue is an instance of its own: its code raises the register pressure of
     // the main loop it shares the kernel with)
-    if (lora && g.qp) hipLaunchKernelGGL((gemm_i8_256<ANIMA_EPI_STORE, false, true, true, true>), grid, block, 0, c->stream, g);
-    else if (lora) hipLaunchKernelGGL((gemm_i8_256<ANIMA_EPI_STORE, false, true, true>), grid, block, 0, c->stream, g);
-    else if (g.qp && w4) hipLaunchKernelGGL((gemm_i8_256<ANIMA_EPI_STORE, true, true, false, true>), grid, block, 0, c->stream, g);
-    else if (g.qp) hipLaunchKernelGGL((gemm_i8_256<ANIMA_EPI_STORE, false, true, false, true>), grid, block, 0, c->stream, g);
-    else if (w4) hipLaunchKernelGGL((gemm_i8_256<ANIMA_EPI_STORE, true, true>), grid, block, 0, c->stream, g);
-    else hipLaunchKernelGGL((gemm_i8_256<ANIMA_EPI_STORE, false, true>), grid, block, 0, c->stream, g);
+    if (lora && g.qp) gemm_i8_launch_t<ANIMA_EPI_STORE, true, true, true>(c, g, tile, w4);
+    else if (lora) gemm_i8_launch_t<ANIMA_EPI_STORE, true, false, true>(c, g, tile, w4);
+    else if (g.qp) gemm_i8_launch_t<ANIMA_EPI_STORE, true, true, false>(c, g, tile, w4);
+    else gemm_i8_launch_t<ANIMA_EPI_STORE, true, false, false>(c, g, tile, w4);
     rc = L.end();
   }
   if (grid8) anima_free(c, grid8);

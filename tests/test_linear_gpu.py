@@ -337,6 +337,32 @@ def test_256_tile_kernel_w4_every_srel(ctx, w4_path, K, path):
     assert np.array_equal(got[rows], orc.linear_epilogue(ref_acc, sx[rows], sw))
 
 
+@pytest.mark.parametrize("M,N,K,kind", [(1, 4, 64, "i8"), (33, 68, 192, "i8"), (256, 2048, 2112, "w4"), (1000, 2052, 2112, "i8"),
+                                        (1537, 2048, 2112, "w4"), (2200, 2052, 2112, "i8"), (2240, 8192, 320, "w4"),
+                                        (7904, 2048, 2112, "i8")])
+def test_int8_tile_sizes(ctx, M, N, K, kind):
+    """Every tile the int8 products choose from, with remainders in rows, columns and k: exact int32 sums, and the
+    fp32 residual epilogue bit for bit ((acc * s_x) * s_w added to C)."""
+    m = amd()
+    case(f"int8 tiles M={M} N={N} K={K} {kind}")
+    rng = np.random.default_rng(M + N + K)
+    q = rng.integers(-127, 128, size=(M, K), dtype=np.int8)
+    sx = rng.uniform(0.5, 1.5, M).astype(np.float32) / 127
+    if kind == "i8":
+        w, s = int8_weight(3, N, K)
+        W = m.weight(m.W_I8, N, K, ctx.upload(w), scale=ctx.upload(s))
+    else:
+        codes, srel, s = w4_weight(3, N, K)
+        w = orc.w4_decode(codes, srel, FIXED_LUT, N, K)
+        W = m.weight(m.W_W4, N, K, ctx.upload(codes), scale=ctx.upload(s), srel=ctx.upload(srel), codebook=ctx.upload(FIXED_LUT))
+    c0 = rng.standard_normal((M, N)).astype(np.float32)
+    out, acc = ctx.upload(c0), ctx.empty((M, N), np.int32)
+    ctx.linear(W, M, out, xq=ctx.upload(q), xs=ctx.upload(sx), epilogue=m.EPI_RESID, acc_out=acc)
+    ref = (q.astype(np.float64) @ w.astype(np.float64).T).astype(np.int32)  # exact: |sums| < 2^53
+    assert np.array_equal(acc.numpy(), ref)
+    assert np.array_equal(out.numpy(), c0 + (ref.astype(np.float32) * sx[:, None]) * s)
+
+
 @pytest.mark.parametrize("act,epi", [("gelu", 0), ("silu", 1)])
 def test_256_tile_kernel_activation_epilogues(ctx, act, epi):
     """The 256x256 kernel with GELU (store) and SiLU (residual add) epilogues at M=4000, N=4100:
