@@ -280,7 +280,8 @@ static int tgemm_launch(anima_ctx* c, const TGemmArgs& p, int amode, int bmode, 
   return L.end();
 }
 
-// ---- conv3x3 on spatial tiles: a workgroup (8 waves) computes a 16 x 32 block of output pixels
+// ---- conv3x3 on spatial tiles (the 3-channel head, and rows of more than 384 channels: what
+// conv3x3_rows_kernel below does not take): a workgroup (8 waves) computes a 16 x 32 block of output pixels
 // for BN = 96 output channels (or one 32-wide column tile when cout <= 32: the 3-channel head).  Per step of 32 input channels the input halo it needs (18 x 34 pixels in
 // output coordinates, sampled through the 2x nearest upsample when up; zero outside the image) and
 // the 9 x 96 x 32 weights are copied once into LDS, so every input value is read from memory once
@@ -431,7 +432,275 @@ __global__ __launch_bounds__(64 * NW) void conv3x3_tile_kernel(TGemmArgs p) {
   }
 }
 
+// ---- conv3x3 by rows: a wave owns 16 output channels x 32 input columns (30 of them with outputs, two
+// halo) and walks the input rows of a strip.  Each input pixel's nine products with the taps,
+// P[ty][tx] = W[ty][tx] . x(y, x), go to the accumulators of the outputs they belong to; the columns'
+// shifts are taken on the finished sums (a neighbouring column is a neighbouring lane: DPP), so the
+// pixels need no halo in LDS and no barrier.  They are read AHEAD 32-channel steps ahead, four
+// consecutive lanes taking 64 contiguous bytes (loads in the operand layout, where consecutive lanes
+// are different pixels, return one lane per cycle and ran at a third of the matrix rate), split, and
+// put into the operand layout through 4 KiB of LDS of the wave's own.  The weights of the workgroup's
+// BN channels stay in LDS (in fragment order) for its whole run; their reads take half the LDS rate.
+// 16 channels and not 32: nine 32 x 32 accumulators leave no second wave per SIMD.
+//
+// Plain: input row y adds P[0] to output row y + 1, P[1] to row y and P[2] to row y - 1, which is then
+// complete: out(x) = A[0](x - 1) + A[1](x) + A[2](x + 1) over its three column accumulators.
+//
+// UP (2x nearest upsample of the input): output pixel (2y + i, 2x + j) reads upsampled row
+// 2y + i + ty - 1, input row y - 1 for (i, ty) = (0, 0), y + 1 for (1, 2) and y otherwise (columns
+// alike): the 36 products of an input pixel's four outputs are sums of only nine distinct ones, a
+// quarter of the matrix work of convolving at the output's resolution (same products):
+//   S[ty][even] = P[ty][0](x - 1) + P[ty][1](x) + P[ty][2](x),  S[ty][odd] = P[ty][0](x) + P[ty][1](x)
+//   + P[ty][2](x + 1);  row 2y = S[0](y - 1) + S[1](y) + S[2](y),  row 2y + 1 = S[0](y) + S[1](y) + S[2](y + 1).
+// Measured against the spatial tiles below (fp32 / bf16, with the channel norms around them): residual
+// block 96 channels 1024 x 1024 1560 -> 1238 / 1303 -> 1074 us, 384 channels 32 x 32 275 -> 97 / 190 ->
+// 73; with the upsampling 192 channels 320 x 448 1120 -> 679 / 814 -> 507, 384 channels 256 x 256
+// 1498 -> 1277 / 971 -> 817 (an upsampling conv of 192 channels at 512 x 512 alone 707 -> 301, a plain
+// one 484 -> 472: about 30% of the matrix rate in both).
+constexpr int CR_COLS = 30, CR_LDS = 110592, CR_WLDS = 4096;  // weights; a wave's pixels
+constexpr int CR_MAXK = CR_LDS / (9 * 2);  // input channels times BN
+
+
+__device__ __forceinline__ f32x4 cr_load(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+  const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
+  return __builtin_bit_cast(f32x4, v);
+}
+// The whole offset in the vector register: with a scalar register as the offset, the compiler lets the
+// next vector instruction overwrite the data of a 16-byte store (no hazard on older chips), and first
+// components of outputs came out wrong here.
+__device__ __forceinline__ void cr_store(__amdgpu_buffer_rsrc_t r, int voff, f32x4 v) {
+  typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, voff, 0, 0);
+}
+
+// v of the column to the left / right; tiles a (columns 0 - 15) and b (16 - 31) in lanes 0 - 15 of a row
+__device__ __forceinline__ float cr_dpp(float old, float v, bool right) {
+  const int o = __builtin_bit_cast(int, old), s = __builtin_bit_cast(int, v);
+  return __builtin_bit_cast(float, right ? __builtin_amdgcn_update_dpp(o, s, 0x101, 0xf, 0xf, false)    // row_shl:1
+                                         : __builtin_amdgcn_update_dpp(o, s, 0x111, 0xf, 0xf, false));  // row_shr:1
+}
+__device__ __forceinline__ float cr_ror(float v, bool right) {
+  const int s = __builtin_bit_cast(int, v);
+  return __builtin_bit_cast(float, right ? __builtin_amdgcn_mov_dpp(s, 0x12f, 0xf, 0xf, false)    // row_ror:15
+                                         : __builtin_amdgcn_mov_dpp(s, 0x121, 0xf, 0xf, false));  // row_ror:1
+}
+
+typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+// eight channels as bf16 hi (+ lo = the rounding's rest), two at a time (packed conversions)
+template <bool SPLIT>
+__device__ __forceinline__ void cr_split(const f32x4 (&v)[2], bf16x8& hi, bf16x8& lo) {
+#pragma unroll
+  for (int e = 0; e < 8; e += 2) {
+    const f32x2_t f = {v[e >> 2][e & 3], v[e >> 2][(e & 3) + 1]};
+    const bf16x2_t h = __builtin_convertvector(f, bf16x2_t);
+    hi[e] = h[0];
+    hi[e + 1] = h[1];
+    if constexpr (SPLIT) {
+      const bf16x2_t l = __builtin_convertvector(f - __builtin_convertvector(h, f32x2_t), bf16x2_t);
+      lo[e] = l[0];
+      lo[e + 1] = l[1];
+    }
+  }
+}
+// orders this wave's LDS accesses for the compiler (the hardware keeps a wave's LDS order)
+__device__ __forceinline__ void cr_order() { asm volatile("" ::: "memory"); }
+
+template <bool UP, bool SPLIT, int BN, int AHEAD>
+__global__ __launch_bounds__(512, 2) void conv3x3_rows_kernel(TGemmArgs p, int R, int ncol, int nstrip, int ncg, int ntask) {
+  __shared__ __attribute__((aligned(16))) char lds[CR_LDS + 8 * CR_WLDS];
+  constexpr int NG = BN / 16, TPW = 8 / NG;  // channel groups; tasks per workgroup
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, l16 = lane & 15, lg = lane >> 4;
+  // an XCD takes all channel blocks of a task one after the other: they read the same pixels
+  const int j8 = blockIdx.x >> 3, cg = j8 % ncg, tg = (blockIdx.x & 7) + 8 * (j8 / ncg);
+  if (tg * TPW >= ntask) return;
+  const int n0 = cg * BN, cin = p.cin, nst = cin / 32;
+  const uint16_t* W = (const uint16_t*)p.b;
+  // weights in fragment order: [32-channel step][tap][channel group][lane: channel lane % 16, k = input
+  // channels 4 (lane / 16) .. + 3 of each half of the step].  (Pixels are then 64 contiguous bytes per
+  // load instruction; eight channels in a row per lane would take twice the segments.)
+#pragma unroll 4
+  for (int u = t; u < nst * 9 * NG * 64; u += 512) {
+    const int ln = u & 63, f = u >> 6, g = f % NG, tap = (f / NG) % 9, st = f / (9 * NG);
+    const int n = min(n0 + 16 * g + (ln & 15), p.N - 1);  // channels past cout: never stored
+    const uint16_t* src = W + (int64_t)n * p.ldb + tap * cin + 32 * st + 4 * (ln >> 4);
+    const uint2 a = *(const uint2*)src, b = *(const uint2*)(src + 16);
+    *(uint4*)(lds + 16 * u) = make_uint4(a.x, a.y, b.x, b.y);
+  }
+  __syncthreads();
+  const int task = tg * TPW + wave / NG, g = wave % NG;
+  if (task >= ntask) return;
+  const int Hin = UP ? p.H >> 1 : p.H, Win = UP ? p.W >> 1 : p.W;
+  const int img = task / (ncol * nstrip), rem = task - img * ncol * nstrip;
+  const int strip = rem / ncol, x0 = (rem - strip * ncol) * CR_COLS;
+  const int y0 = strip * R, y1 = min(y0 + R, Hin);
+  const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.a + (int64_t)img * Hin * Win * cin), (short)0, Hin * Win * cin * 4, 0x00020000);
+  const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)(p.c + (int64_t)img * p.H * p.W * p.ldc), (short)0, p.H * p.W * (int)p.ldc * 4, 0x00020000);
+  const int n = n0 + 16 * g + 4 * lg;  // this lane's four channels
+  // this lane's pixel of each tile, as read (pixel lane / 4, channels 4 (lane % 4) .. + 3 of each half of
+  // the step) and as multiplied and written: columns outside the image read zeros past the resource,
+  // halo lanes' loads of the output read zeros and their stores are dropped
+  int xo[2], oo[2];
+#pragma unroll
+  for (int i = 0; i < 2; i++) {
+    const int xr = x0 - 1 + 16 * i + (lane >> 2), lx = 16 * i + l16, x = x0 - 1 + lx;
+    xo[i] = xr >= 0 && xr < Win ? (xr * cin + 4 * (lane & 3)) * 4 : 0x7ffffff0;
+    oo[i] = lx >= 1 && lx <= CR_COLS && x < Win && n < p.N ? ((UP ? 2 * x : x) * (int)p.ldc + n) * 4 : 0x7fff0000;
+  }
+  f32x4 raw[AHEAD][2][2];  // slot d: the next step d, d + AHEAD, ... of a row (nst % AHEAD == 0)
+  auto load = [&](int y, int st, f32x4 (&v)[2][2]) __attribute__((always_inline)) {
+    const int so = (min(max(y, 0), Hin - 1) * Win * cin + 32 * st) * 4;
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      v[i][0] = cr_load(rx, xo[i], so);
+      v[i][1] = cr_load(rx, xo[i], so + 64);
+    }
+  };
+  const char* wl = lds + (g * 64 + lane) * 16;
+  // pixel a, channel group b of a tile at slot 4 a + (b ^ (a / 4)): both sides' accesses are conflict-free
+  char* const px = lds + CR_LDS + wave * CR_WLDS;
+  char* const pw = px + 16 * (4 * (lane >> 2) + ((lane & 3) ^ (lane >> 4)));
+  const char* const pr = px + 16 * (4 * l16 + (lg ^ (l16 >> 2)));
+  f32x4 bias = {};
+  if (p.bias && n < p.N)
+#pragma unroll
+    for (int r = 0; r < 4; r++) bias[r] = p.bias[n + r];
+  const int row_bytes = p.W * (int)p.ldc * 4;  // of the output
+
+  // UP: the row's products P, and the previous row's S[0] and S[0] + S[1] ([tile][even, odd]).
+  // Plain: P[3 ty + tx] are the column accumulators of output row y + 1 - ty.
+  f32x4 P[9][2], c0[2][2] = {}, c01[2][2] = {};
+#pragma unroll
+  for (int k = 0; k < 9; k++) P[k][0] = P[k][1] = f32x4{};
+#pragma unroll
+  for (int d = 0; d < AHEAD; d++) load(y0 - 1, d, raw[d]);
+  for (int y = y0 - 1; y <= y1; y++) {
+    f32x4 res[2] = {};
+    if (!UP && p.resid && y > y0)
+#pragma unroll
+      for (int i = 0; i < 2; i++) res[i] = cr_load(ro, oo[i] + (y - 1) * row_bytes, 0);
+    if (y >= 0 && y < Hin) {
+      for (int st = 0; st < nst; st += AHEAD)
+#pragma unroll
+        for (int d = 0; d < AHEAD; d++) {
+          bf16x8 hi[2], lo[2];
+#pragma unroll
+          for (int i = 0; i < 2; i++) {
+            cr_split<SPLIT>(raw[d][i], hi[i], lo[i]);
+            *(bf16x8*)(pw + 1024 * i) = hi[i];
+            if constexpr (SPLIT) *(bf16x8*)(pw + 2048 + 1024 * i) = lo[i];
+          }
+          cr_order();
+#pragma unroll
+          for (int i = 0; i < 2; i++) {
+            hi[i] = *(const bf16x8*)(pr + 1024 * i);
+            if constexpr (SPLIT) lo[i] = *(const bf16x8*)(pr + 2048 + 1024 * i);
+          }
+          cr_order();
+          if (st + d + AHEAD < nst) load(y, st + d + AHEAD, raw[d]);
+          else load(y + 1, d, raw[d]);
+          const char* ws = wl + (st + d) * (9 * NG * 1024);
+          // three taps at a time, so that a product and the next one on its accumulator are six apart
+#pragma unroll
+          for (int ty = 0; ty < 3; ty++) {
+            bf16x8 w[3];
+#pragma unroll
+            for (int tx = 0; tx < 3; tx++) w[tx] = *(const bf16x8*)(ws + (3 * ty + tx) * (NG * 1024));
+#pragma unroll
+            for (int q = 0; q < 6; q++)
+              P[3 * ty + q / 2][q & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[q / 2], hi[q & 1], P[3 * ty + q / 2][q & 1], 0, 0, 0);
+            if constexpr (SPLIT)
+#pragma unroll
+              for (int q = 0; q < 6; q++)
+                P[3 * ty + q / 2][q & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[q / 2], lo[q & 1], P[3 * ty + q / 2][q & 1], 0, 0, 0);
+          }
+        }
+    } else {
+#pragma unroll
+      for (int d = 0; d < AHEAD; d++) load(y + 1, d, raw[d]);
+    }
+    if constexpr (!UP) {
+      if (y > y0) {  // output row y - 1
+        f32x4 o[2];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float a0 = P[6][0][r], a1 = P[6][1][r], b0 = P[8][0][r], b1 = P[8][1][r];
+          o[0][r] = (cr_dpp(0.0f, a0, false) + P[7][0][r]) + cr_dpp(cr_ror(b1, true), b0, true);
+          o[1][r] = (cr_dpp(cr_ror(a0, false), a1, false) + P[7][1][r]) + cr_dpp(0.0f, b1, true);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; i++) cr_store(ro, oo[i] + (y - 1) * row_bytes, res[i] + (o[i] + bias));
+      }
+#pragma unroll
+      for (int k = 8; k >= 3; k--) P[k][0] = P[k - 3][0], P[k][1] = P[k - 3][1];
+#pragma unroll
+      for (int k = 0; k < 3; k++) P[k][0] = P[k][1] = f32x4{};
+    } else {
+      // S of one kernel row: [tile][even, odd].  Rows 2, 1, 0 in turn, so that each row's products are
+      // dead before the next row's sums are formed.
+      const auto sums = [&](int ty, f32x4 (&S)[2][2]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const float l0 = P[3 * ty][0][r], l1 = P[3 * ty][1][r], r0 = P[3 * ty + 2][0][r], r1 = P[3 * ty + 2][1][r];
+          const float m0 = P[3 * ty + 1][0][r], m1 = P[3 * ty + 1][1][r];
+          const float left0 = cr_dpp(0.0f, l0, false), left1 = cr_dpp(cr_ror(l0, false), l1, false);
+          const float right0 = cr_dpp(cr_ror(r1, true), r0, true), right1 = cr_dpp(0.0f, r1, true);
+          S[0][0][r] = left0 + (m0 + r0);
+          S[0][1][r] = (l0 + m0) + right0;
+          S[1][0][r] = left1 + (m1 + r1);
+          S[1][1][r] = (l1 + m1) + right1;
+        }
+      };
+      const auto put = [&](int i, int e, int row, f32x4 v) __attribute__((always_inline)) {
+        const int vo = oo[i] + row * row_bytes + e * (int)p.ldc * 4;
+        v = v + bias;
+        if (p.resid) v = cr_load(ro, vo, 0) + v;
+        cr_store(ro, vo, v);
+      };
+      f32x4 S2[2][2], S1[2][2];
+      sums(2, S2);
+      if (y > y0)  // the odd row of y - 1
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int e = 0; e < 2; e++) put(i, e, 2 * y - 1, c01[i][e] + S2[i][e]);
+      __builtin_amdgcn_sched_barrier(0);
+      sums(1, S1);
+      if (y >= y0 && y < y1)
+#pragma unroll
+        for (int i = 0; i < 2; i++)
+#pragma unroll
+          for (int e = 0; e < 2; e++) put(i, e, 2 * y, c0[i][e] + (S1[i][e] + S2[i][e]));
+      __builtin_amdgcn_sched_barrier(0);
+      sums(0, c0);
+#pragma unroll
+      for (int i = 0; i < 2; i++)
+#pragma unroll
+        for (int e = 0; e < 2; e++) c01[i][e] = c0[i][e] + S1[i][e];
+#pragma unroll
+      for (int k = 0; k < 9; k++) P[k][0] = P[k][1] = f32x4{};
+    }
+  }
+}
+
 static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
+
+// Rows per strip of conv3x3_rows_kernel: an XCD's workgroups run in rounds of one per CU, and each
+// takes R + 2 rows' products.  Returns the cost, rounds * (R + 2).
+static int64_t conv3x3_rows_strip(int num_cus, int64_t cols, int Hin, int ncg, int tpw, int* R) {
+  const int64_t cus = num_cus >= 8 ? num_cus / 8 : 1;
+  int64_t bc = -1;
+  for (int r = 1; r <= 256 && r <= Hin; r++) {
+    const int64_t ntg = (cols * ((Hin + r - 1) / r) + tpw - 1) / tpw, wgs = (ntg + 7) / 8 * ncg, cost = (wgs + cus - 1) / cus * (r + 2);
+    if (bc < 0 || cost <= bc) {
+      bc = cost;
+      *R = r;
+    }
+  }
+  return bc;
+}
 
 int conv3x3_launch(anima_ctx* c, const anima_conv_desc* d) {
   if (!d) return fail(c, ANIMA_E_ARG, "anima_conv3x3: null descriptor");
@@ -463,6 +732,45 @@ int conv3x3_launch(anima_ctx* c, const anima_conv_desc* d) {
   p.N = d->cout;
   p.K = 9 * d->cin;
   const bool split = d->precision == ANIMA_PREC_FP32;
+  // conv by rows: weights of 32 (or 16) output channels in LDS, 16-byte stores of four channels, 32-bit
+  // offsets into an image
+  const int Hin = d->up ? d->H / 2 : d->H, Win = d->up ? d->W / 2 : d->W;
+  const int64_t in_bytes = (int64_t)Hin * Win * d->cin * 4, out_bytes = (int64_t)d->H * d->W * d->cout * 4;
+  if (d->cin % 32 == 0 && d->cin * 16 <= CR_MAXK && d->cout % 4 == 0 && d->cout <= 4096 && al16(d->out) &&
+      in_bytes < (1LL << 31) - 65536 && out_bytes < (1LL << 31) - 65536) {
+    const int bn = d->cin * 32 <= CR_MAXK && d->cout > 16 ? 32 : 16, tpw = 8 / (bn / 16);
+    const int ncol = (Win + CR_COLS - 1) / CR_COLS, ncg = (d->cout + bn - 1) / bn;
+    int R = 1;
+    conv3x3_rows_strip(c->num_cus, (int64_t)d->B * ncol, Hin, ncg, tpw, &R);
+    const int nstrip = (Hin + R - 1) / R;
+    const int64_t ntask = (int64_t)d->B * ncol * nstrip, ntg = (ntask + tpw - 1) / tpw, blocks = (ntg + 7) / 8 * 8 * ncg;
+    if (ntask <= 0x7ffffff && blocks <= 0x7fffffff) {
+      const dim3 grid((unsigned)blocks);
+      Launch L(c, d->up ? "conv3x3.up" : "conv3x3", 2.0 * M * d->cout * 9.0 * d->cin, 0.0);
+#define CRA(U, S, BN, A) hipLaunchKernelGGL((conv3x3_rows_kernel<U, S, BN, A>), grid, dim3(512), 0, c->stream, p, R, ncol, nstrip, ncg, (int)ntask)
+#define CRB(U, S, BN)                     \
+  {                                       \
+    if (d->cin % 96 == 0) CRA(U, S, BN, 3); \
+    else CRA(U, S, BN, 1);                \
+  }
+#define CRU(S, BN)              \
+  {                             \
+    if (d->up) CRB(true, S, BN) \
+    else CRB(false, S, BN)      \
+  }
+      if (bn == 32) {
+        if (split) CRU(true, 32)
+        else CRU(false, 32)
+      } else {
+        if (split) CRU(true, 16)
+        else CRU(false, 16)
+      }
+#undef CRU
+#undef CRB
+#undef CRA
+      return L.end();
+    }
+  }
   const int bn = d->cout % 96 == 0 ? 96 : d->cout <= 32 ? 32 : 0;  // 96-channel tiles, or one 32-wide tile
   if (bn && d->cin % CT_CC == 0 && d->H % CT_TH == 0 && d->W % CT_TW == 0 &&
       (int64_t)d->B * (d->H / CT_TH) * (d->W / CT_TW) <= 0x7fffffff && (d->cout + bn - 1) / bn <= 65535) {

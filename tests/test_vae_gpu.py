@@ -68,6 +68,15 @@ CONV_CASES = [  # B, H, W (output), cin, cout, up, resid
     (1, 16, 32, 384, 384, False, False),
     (1, 16, 32, 96, 3, False, True),  # one 32-wide column tile for 3 channels (the head)
     (1, 32, 64, 64, 32, True, False),
+    # the upsampling conv at input resolution: one pixel, strips and 30-column tiles with remainders, several
+    # images, channels that are no multiple of 16, and what it leaves to the output-resolution kernels
+    (1, 2, 2, 32, 4, True, False),
+    (2, 62, 126, 64, 36, True, True),
+    (3, 60, 120, 32, 20, True, False),
+    (1, 10, 62, 288, 48, True, True),
+    (1, 36, 60, 512, 8, True, False),
+    (1, 12, 12, 48, 8, True, False),
+    (1, 12, 12, 32, 6, True, False),
 ]
 
 
