@@ -1044,11 +1044,346 @@ __global__ __launch_bounds__(256) void pv_sum_kernel(const float* part, int ks, 
   o[m * ldo + (i - m * D)] = acc * rl[m];
 }
 
+// ---- attention of 384-dim heads (the VAE decoder's single head over all latent positions), fused
+//
+// The chunked path writes the score matrix (1 GiB at 128 x 128 latents), reads and rewrites it for the
+// softmax and reads it again; here scores live in registers.  Bound by the matrix cores (with SPLIT
+// three bf16 products per score and per output, as on the chunked path: hi.hi + lo.hi + hi.lo).  A
+// pass first writes K and V as bf16 planes in MFMA fragment order, per block of 32 keys: K as
+// [16-dim step][plane][lane][8 dims], V^T as [32-dim tile][16-key step][plane][lane][8 keys], 1 KiB
+// per fragment, so that the main loop's copies and LDS reads are linear.  A workgroup is 128 queries,
+// 8 waves: waves w and w + 4 share 32 queries and split the 384 dims (queries, and outputs, of 192 dims
+// take 96 registers each with SPLIT; all 384 in one wave per SIMD spilled and overlapped nothing).
+// Each takes half of the score products; the halves are exchanged through LDS.  A block's weights are
+// formed beside the next block's score products.  K and V go through one LDS slot each, copied one
+// phase ahead.  Scores are computed transposed (a lane holds one query's keys), so a row's softmax
+// needs one lane exchange, and its weights are the next product's operand as they stand (V^T's keys
+// are stored in that order: 0-3, 8-11, 4-7, 12-15 of each 16).  Queries too few for the CUs split the
+// keys, partial outputs (unnormalized, with the row's maximum and sum) combined afterwards.
+// 128 x 128 latents, fp32: FIGURES
+constexpr int FA_D = 384, FA_KB = 32, FA_Q = 128, FA_NS = FA_D / 16, FA_NT = FA_D / 32, FA_MAXB = 64;
+
+struct FaArgs {
+  const float *q, *k, *v;
+  float* o;
+  int64_t ldq, ldk, ldv, ldo, qbs, kbs, vbs, obs;  // rows, batch strides (offsets applied)
+  char* kv;       // prepared blocks [B][Hkv][nkb][K, V]
+  float* part;    // partial outputs [item][split][128][384], then (maximum, sum) [item][split][128][2]
+  float* ml;
+  int64_t kv_head;  // bytes of one (batch, kv head) of kv
+  int Lq, H, group, nkb, nqt, splits, per;  // per: key blocks per split
+  float c;          // scale * log2(e)
+  int valid[FA_MAXB];
+};
+
+// bf16 hi (and the rest lo) of 8 values
+template <bool SPLIT>
+__device__ __forceinline__ void fa_split(const float (&v)[8], bf16x8& hi, bf16x8& lo) {
+  cr_split<SPLIT>({f32x4{v[0], v[1], v[2], v[3]}, f32x4{v[4], v[5], v[6], v[7]}}, hi, lo);
+}
+
+// One block of 32 keys of one kv head: K and V rows to fragments (keys past the valid ones as zeros).
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void attn384_prep_kernel(FaArgs a) {
+  constexpr int NP = SPLIT ? 2 : 1;
+  __shared__ float vs[FA_KB][FA_D + 1];
+  const int t = threadIdx.x, kb = blockIdx.x, hk = blockIdx.y, b = blockIdx.z, k0 = kb * FA_KB;
+  const int nv = min(FA_KB, a.valid[b] - k0);  // may be <= 0: a block of zeros
+  const float* K = a.k + (int64_t)b * a.kbs + (int64_t)hk * FA_D;
+  const float* V = a.v + (int64_t)b * a.vbs + (int64_t)hk * FA_D;
+  char* out = a.kv + ((int64_t)b * gridDim.y + hk) * a.kv_head + (int64_t)kb * (2 * FA_NS * NP * 1024);
+  for (int u = t; u < FA_KB * FA_D / 4; u += 256) {
+    const int r = u / (FA_D / 4), d = 4 * (u % (FA_D / 4));
+    const f32x4 x = r < nv ? *(const f32x4*)(V + (int64_t)(k0 + r) * a.ldv + d) : f32x4{};
+#pragma unroll
+    for (int e = 0; e < 4; e++) vs[r][d + e] = x[e];
+  }
+  for (int u = t; u < FA_KB * FA_D / 8; u += 256) {
+    const int r = u / (FA_D / 8), pc = u % (FA_D / 8);  // row, piece of 8 dims: step pc / 2, half pc % 2
+    f32x4 x[2] = {};
+    if (r < nv) {
+      const float* src = K + (int64_t)(k0 + r) * a.ldk + 8 * pc;
+      x[0] = *(const f32x4*)src;
+      x[1] = *(const f32x4*)(src + 4);
+    }
+    bf16x8 hi, lo;
+    cr_split<SPLIT>(x, hi, lo);
+    char* dst = out + (pc >> 1) * (NP * 1024) + (r + 32 * (pc & 1)) * 16;
+    *(bf16x8*)dst = hi;
+    if constexpr (SPLIT) *(bf16x8*)(dst + 1024) = lo;
+  }
+  __syncthreads();
+  out += FA_NS * NP * 1024;
+  for (int u = t; u < FA_NT * 2 * 64; u += 256) {
+    const int ln = u & 63, f = u >> 6, tile = f >> 1, s2 = f & 1, d = 32 * tile + (ln & 31), hf = ln >> 5;
+    float x[8];
+#pragma unroll
+    for (int j = 0; j < 8; j++) x[j] = vs[16 * s2 + 4 * hf + (j & 3) + 8 * (j >> 2)][d];
+    bf16x8 hi, lo;
+    fa_split<SPLIT>(x, hi, lo);
+    char* dst = out + f * (NP * 1024) + ln * 16;
+    *(bf16x8*)dst = hi;
+    if constexpr (SPLIT) *(bf16x8*)(dst + 1024) = lo;
+  }
+}
+
+typedef __attribute__((address_space(3))) void fa_lds_t;
+__device__ __forceinline__ void fa_copy(__amdgpu_buffer_rsrc_t r, char* dst, int voff, int soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (fa_lds_t*)dst, 16, voff, soff, 0, 0);
+}
+// this wave's copies have landed and its LDS accesses are done; then every wave's
+__device__ __forceinline__ void fa_wait_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(7 << 4);  // vmcnt(0), lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <bool SPLIT>
+__global__ __launch_bounds__(512, 2) void attn384_kernel(FaArgs a, int nitem) {
+  constexpr int NP = SPLIT ? 2 : 1, TB = FA_NS * NP * 1024, CPW = TB / 8192;  // bytes of a K (V) block; copies per wave
+  constexpr int HS = FA_NS / 2, HT = FA_NT / 2;                              // 16-dim steps, 32-dim tiles of a wave
+  __shared__ __attribute__((aligned(1024))) char smem[2 * TB + 2 * 8 * 4096];
+  const int t = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(t >> 6), lane = t & 63, lq = lane & 31, hf = lane >> 5;
+  const int u = wave >> 2;  // dims 192 u .. + 191 of the queries of wave % 4
+  // items [batch, head][split][query tile]: an XCD's contiguous range shares K / V streams in its L2
+  const int it = xcd_remap(blockIdx.x, nitem);
+  const int bh = it / (a.splits * a.nqt), rem = it - bh * a.splits * a.nqt, sp = rem / a.nqt, qt = rem - sp * a.nqt;
+  const int b = bh / a.H, h = bh - b * a.H;
+  const int valid = a.valid[b], nkb = (valid + FA_KB - 1) / FA_KB;
+  const int kb0 = sp * a.per, nb = min(a.per, nkb - kb0);  // may be <= 0 for a shorter batch element
+  const int row = qt * FA_Q + 32 * (wave & 3) + lq;
+
+  f32x16 O[HT];
+#pragma unroll
+  for (int i = 0; i < HT; i++) O[i] = f32x16{};
+  float m = -INFINITY, l = 0.0f;
+
+  if (nb > 0) {
+    const char* src = a.kv + ((int64_t)b * (a.H / a.group) + h / a.group) * a.kv_head + (int64_t)kb0 * (2 * TB);
+    const __amdgpu_buffer_rsrc_t rk = __builtin_amdgcn_make_buffer_rsrc((void*)src, (short)0, 2 * nb * TB, 0x00020000);
+    // K blocks go through the first slot, V blocks through the second; block 2 j (+ 1) of the stream
+    auto issue = [&](int blk) __attribute__((always_inline)) {
+      char* dst = smem + (blk & 1) * TB + wave * (CPW * 1024);
+#pragma unroll
+      for (int c = 0; c < CPW; c++) fa_copy(rk, dst + c * 1024, (wave * CPW + c) * 1024 + lane * 16, blk * TB);
+    };
+    issue(0);
+    bf16x8 qh[HS], ql[SPLIT ? HS : 1];
+    {
+      const float* Q = a.q + (int64_t)b * a.qbs + (int64_t)min(row, a.Lq - 1) * a.ldq + (int64_t)h * FA_D + 192 * u + 8 * hf;
+#pragma unroll
+      for (int s = 0; s < HS; s++) {
+        const f32x4 x[2] = {*(const f32x4*)(Q + 16 * s), *(const f32x4*)(Q + 16 * s + 4)};
+        bf16x8 lo;
+        cr_split<SPLIT>(x, qh[s], lo);
+        if constexpr (SPLIT) ql[s] = lo;
+      }
+    }
+    const char* const kp = smem + u * (HS * NP * 1024) + lane * 16;
+    const char* const vp = smem + TB + u * (2 * HT * NP * 1024) + lane * 16;
+    // this wave's partial scores and its partner's, [quad][lane], of even and odd blocks
+    char* const xo = smem + 2 * TB + wave * 4096 + lane * 16;
+    const char* const xi = smem + 2 * TB + (wave ^ 4) * 4096 + lane * 16;
+    auto scores = [&](f32x16& S) __attribute__((always_inline)) {
+#pragma unroll
+      for (int s = 0; s < HS; s++) {
+        const bf16x8 kh = *(const bf16x8*)(kp + s * (NP * 1024));
+        S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, qh[s], S, 0, 0, 0);
+        if constexpr (SPLIT) {
+          const bf16x8 kl = *(const bf16x8*)(kp + s * (NP * 1024) + 1024);
+          S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kh, ql[s], S, 0, 0, 0);
+          S = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kl, qh[s], S, 0, 0, 0);
+        }
+      }
+    };
+    auto give = [&](const f32x16& S, int j) __attribute__((always_inline)) {
+#pragma unroll
+      for (int q = 0; q < 4; q++)
+        *(f32x4*)(xo + (j & 1) * 32768 + q * 1024) = f32x4{S[4 * q], S[4 * q + 1], S[4 * q + 2], S[4 * q + 3]};
+    };
+    fa_wait_barrier();
+    f32x16 S = {};
+    scores(S);
+    give(S, 0);
+    fa_wait_barrier();
+    if (nb > 1) issue(2);
+    for (int j = 0; j < nb; j++) {
+      fa_wait_barrier();  // K j + 1 and the scores of j are there; V j - 1 has been read
+      issue(2 * j + 1);
+      // scores times c, keys past the valid ones out; register r is key 8 (r / 4) + 4 hf + r % 4
+      float y[16];
+      const int left = valid - (kb0 + j) * FA_KB;
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const f32x4 x = *(const f32x4*)(xi + (j & 1) * 32768 + q * 1024);
+#pragma unroll
+        for (int e = 0; e < 4; e++) y[4 * q + e] = (S[4 * q + e] + x[e]) * a.c;
+      }
+      if (left < FA_KB)
+#pragma unroll
+        for (int r = 0; r < 16; r++) y[r] = 8 * (r >> 2) + 4 * hf + (r & 3) < left ? y[r] : -INFINITY;
+      float mx = y[0];
+#pragma unroll
+      for (int r = 1; r < 16; r++) mx = fmaxf(mx, y[r]);
+      mx = fmaxf(mx, __shfl_xor(mx, 32));
+      if (__any(mx > m)) {  // (rare once the first blocks are done)
+        const float mn = fmaxf(m, mx), al = __builtin_amdgcn_exp2f(m - mn);
+        m = mn;
+        l = l * al;
+#pragma unroll
+        for (int i = 0; i < HT; i++) O[i] = O[i] * al;
+      }
+      // the next block's scores beside this block's weights (after the last block: of the last again, unused)
+      S = f32x16{};
+      scores(S);
+      bf16x8 ph[2], pl[2];
+#pragma unroll
+      for (int s2 = 0; s2 < 2; s2++) {
+        float e[8];
+#pragma unroll
+        for (int r = 0; r < 8; r++) {
+          e[r] = __builtin_amdgcn_exp2f(y[8 * s2 + r] - m);
+          l += e[r];
+        }
+        fa_split<SPLIT>(e, ph[s2], pl[s2]);
+      }
+      give(S, j + 1);
+      fa_wait_barrier();  // V j is there; K j + 1 has been read
+      if (j + 2 < nb) issue(2 * j + 4);
+#pragma unroll
+      for (int f = 0; f < 2 * HT; f++) {  // tile f / 2, keys 16 (f % 2) .. + 15
+        const bf16x8 vh = *(const bf16x8*)(vp + f * NP * 1024);
+        f32x16& o = O[f >> 1];
+        o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, ph[f & 1], o, 0, 0, 0);
+        if constexpr (SPLIT) {
+          const bf16x8 vl = *(const bf16x8*)(vp + f * NP * 1024 + 1024);
+          o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vh, pl[f & 1], o, 0, 0, 0);
+          o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vl, ph[f & 1], o, 0, 0, 0);
+        }
+      }
+    }
+  }
+  l = l + __shfl_xor(l, 32);
+  float* dst;
+  float f = 1.0f;
+  if (a.splits == 1) {
+    if (row >= a.Lq) return;
+    dst = a.o + (int64_t)b * a.obs + (int64_t)row * a.ldo + (int64_t)h * FA_D;
+    f = 1.0f / l;
+  } else {
+    const int64_t pr = ((int64_t)bh * a.splits + sp) * a.nqt * FA_Q + row;
+    dst = a.part + pr * FA_D;
+    if (hf == 0 && u == 0) {
+      a.ml[2 * pr] = m;
+      a.ml[2 * pr + 1] = l;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < HT; i++)
+#pragma unroll
+    for (int q = 0; q < 4; q++) {
+      const f32x4 v = {O[i][4 * q] * f, O[i][4 * q + 1] * f, O[i][4 * q + 2] * f, O[i][4 * q + 3] * f};
+      *(f32x4*)(dst + 192 * u + 32 * i + 8 * q + 4 * hf) = v;
+    }
+}
+
+// out = sum_z 2^(m_z - M) O_z / sum_z 2^(m_z - M) l_z, M = max m_z: 96 threads (4 dims each) per row.
+__global__ __launch_bounds__(192) void attn384_combine_kernel(FaArgs a) {
+  const int row = blockIdx.x * 2 + threadIdx.x / 96, d = 4 * (threadIdx.x % 96), bh = blockIdx.y;
+  if (row >= a.Lq) return;
+  const int64_t st = (int64_t)a.nqt * FA_Q, pr = (int64_t)bh * a.splits * st + row;
+  float M = -INFINITY;
+  for (int z = 0; z < a.splits; z++) M = fmaxf(M, a.ml[2 * (pr + z * st)]);
+  f32x4 acc = {};
+  float l = 0.0f;
+  for (int z = 0; z < a.splits; z++) {
+    const float lz = a.ml[2 * (pr + z * st) + 1];
+    if (lz == 0.0f) continue;  // a split past this batch element's keys
+    const float w = __builtin_amdgcn_exp2f(a.ml[2 * (pr + z * st)] - M);
+    acc = acc + *(const f32x4*)(a.part + (pr + z * st) * FA_D + d) * w;
+    l = l + lz * w;
+  }
+  const int b = bh / a.H, h = bh - b * a.H;
+  *(f32x4*)(a.o + (int64_t)b * a.obs + (int64_t)row * a.ldo + (int64_t)h * FA_D + d) = acc * (1.0f / l);
+}
+
+// 384-dim heads without a causal mask, where the operands and partial outputs stay below 1 GiB of
+// workspace (the chunked path's own bound on scores): returns 1 if launched, 0 if not taken, or an error.
+static int attention384_launch(anima_ctx* c, const anima_attn_desc* d, const int* kv_len) {
+  if (d->D != FA_D || d->causal || d->B > FA_MAXB) return 0;
+  const int group = d->group <= 0 ? 1 : d->group, Hk = d->H / group;
+  const bool split = d->precision == ANIMA_PREC_FP32;
+  FaArgs a{};
+  int vmax = 0;
+  for (int b = 0; b < d->B; b++) {
+    if (kv_len[b] < 1) return 0;
+    a.valid[b] = kv_len[b];
+    vmax = std::max(vmax, kv_len[b]);
+  }
+  a.nkb = (vmax + FA_KB - 1) / FA_KB;
+  a.nqt = (d->Lq + FA_Q - 1) / FA_Q;
+  const int64_t bh = (int64_t)d->B * d->H, wgs = bh * a.nqt;
+  // key splits: rounds of one workgroup per CU times its key blocks (and about three blocks' time of
+  // prologue and stores, and each split's share of the combining pass), splits of at least 4 blocks
+  int64_t best = -1;
+  for (int s = 1; s <= 16 && (s == 1 || a.nkb / s >= 4); s++) {
+    const int64_t cost = (wgs * s + c->num_cus - 1) / c->num_cus * ((a.nkb + s - 1) / s + 3) + (s > 1 ? s : 0);
+    if (best < 0 || cost < best) {
+      best = cost;
+      a.splits = s;
+    }
+  }
+  a.per = (a.nkb + a.splits - 1) / a.splits;
+  a.splits = (a.nkb + a.per - 1) / a.per;
+  const int64_t tb = (int64_t)FA_NS * (split ? 2 : 1) * 1024, rows = a.splits > 1 ? bh * a.splits * a.nqt * FA_Q : 0;
+  a.kv_head = 2 * tb * a.nkb;
+  const int64_t kv_bytes = a.kv_head * d->B * Hk, bytes = kv_bytes + rows * (FA_D + 2) * 4;
+  if (a.kv_head >= (1LL << 31) || bytes > (1LL << 30) || wgs * a.splits > 0x7fffffff || bh > 65535 || Hk > 65535) return 0;
+  void* ws = nullptr;
+  int rc = workspace(c, (size_t)bytes, &ws);
+  if (rc) return 0;  // (the chunked path asks for its own amount)
+  a.q = d->q + d->q_off;
+  a.k = d->k + d->k_off;
+  a.v = d->v + d->v_off;
+  a.o = d->o + d->o_off;
+  a.ldq = d->ldq, a.ldk = d->ldk, a.ldv = d->ldv, a.ldo = d->ldo;
+  a.qbs = d->q_bstride, a.kbs = d->k_bstride, a.vbs = d->v_bstride, a.obs = d->o_bstride;
+  a.kv = (char*)ws;
+  a.part = (float*)((char*)ws + kv_bytes);
+  a.ml = a.part + rows * FA_D;
+  a.Lq = d->Lq;
+  a.H = d->H;
+  a.group = group;
+  a.c = (d->scale != 0.0f ? d->scale : 1.0f / sqrtf((float)FA_D)) * 1.4426950408889634f;
+  {
+    Launch L(c, "attn.384.prep", 0.0, 8.0 * d->B * Hk * vmax * FA_D * 2);
+    const dim3 grid(a.nkb, Hk, d->B);
+    if (split) hipLaunchKernelGGL(attn384_prep_kernel<true>, grid, dim3(256), 0, c->stream, a);
+    else hipLaunchKernelGGL(attn384_prep_kernel<false>, grid, dim3(256), 0, c->stream, a);
+    if ((rc = L.end())) return rc;
+  }
+  {
+    Launch L(c, "attn.384", 4.0 * bh * d->Lq * (double)vmax * FA_D, 0.0);
+    const int n = (int)(wgs * a.splits);
+    if (split) hipLaunchKernelGGL(attn384_kernel<true>, dim3(n), dim3(512), 0, c->stream, a, n);
+    else hipLaunchKernelGGL(attn384_kernel<false>, dim3(n), dim3(512), 0, c->stream, a, n);
+    if ((rc = L.end())) return rc;
+  }
+  if (a.splits > 1) {
+    Launch L(c, "attn.384.combine", 0.0, 4.0 * rows * FA_D);
+    hipLaunchKernelGGL(attn384_combine_kernel, dim3((d->Lq + 1) / 2, (unsigned)bh), dim3(192), 0, c->stream, a);
+    if ((rc = L.end())) return rc;
+  }
+  return 1;
+}
+
 int attention_chunked_launch(anima_ctx* c, const anima_attn_desc* d, const int* kv_len) {
   const int group = d->group <= 0 ? 1 : d->group;
   const int D = d->D, Lq = d->Lq, Lk = d->Lk;
   const float scale = d->scale != 0.0f ? d->scale : 1.0f / sqrtf((float)D);
   const bool split = d->precision == ANIMA_PREC_FP32;
+  if (const int r384 = attention384_launch(c, d, kv_len)) return r384 < 0 ? r384 : ANIMA_OK;
   // score rows per chunk: at most 1 GiB of scores (one chunk for the VAE's 16384 tokens at 1024x1024;
   // the device has 288 GB), a multiple of the 128-row tile
   int64_t rows = std::max<int64_t>(TG_BM, ((int64_t)(1 << 30) / 4 / Lk) / TG_BM * TG_BM);

@@ -114,6 +114,12 @@ ATTN_CASES = [  # B, Lq, Lk, H, group, D, kv_len
     (2, 256, 200, 2, 2, 384, [200, 77]),
     (1, 2304, 16384, 1, 1, 384, None),  # one 2304 x 16384 score chunk
     (1, 96, 150, 3, 1, 96, None),
+    # the fused 384-dim kernel: one query and key, one block and its edges, key splits with remainders and
+    # batch elements shorter than a split
+    (1, 1, 1, 1, 1, 384, None),
+    (1, 129, 32, 1, 1, 384, None),
+    (1, 127, 33, 2, 1, 384, None),
+    (3, 200, 1000, 2, 2, 384, [1000, 31, 545]),
 ]
 
 
