@@ -56,6 +56,37 @@ __global__ __launch_bounds__(256) void rmsnorm_kernel(const float* X, const floa
   for (int c = lane; c < cols; c += 64) y[c] = x[c] * r * W[c];
 }
 
+// The same sums in the same order with the row held in registers (64 NV >= cols): every load of the
+// row and its weights is in flight at once, where the loop above waits for one load at a time (one row
+// of 2048: 18.8 us; 43 rows of 1024: 11 us; here 3.8 and 3.9).  Columns past the row read as zero
+// (adding 0 is exact).
+template <int NV>
+__global__ __launch_bounds__(256) void rmsnorm_reg_kernel(const float* X, const float* W, float* Y, int64_t rows, int cols,
+                                                          float eps) {
+  const int lane = threadIdx.x & 63;
+  const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+  if (row >= rows) return;
+  const float* x = X + row * cols;
+  float v[NV], w[NV];
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const int c = lane + 64 * i;
+    v[i] = c < cols ? x[c] : 0.0f;
+    w[i] = c < cols ? W[c] : 0.0f;
+  }
+  float ss = 0.0f;
+#pragma unroll
+  for (int i = 0; i < NV; i++) ss += v[i] * v[i];
+  ss = tree_sum_down(ss, 64);
+  const float r = 1.0f / sqrtf(__shfl(ss, 0) / (float)cols + eps);
+  float* y = Y + row * cols;
+#pragma unroll
+  for (int i = 0; i < NV; i++) {
+    const int c = lane + 64 * i;
+    if (c < cols) y[c] = v[i] * r * w[i];
+  }
+}
+
 // One thread per rotated pair (app/gpu/kernels.js:343-356).
 __global__ __launch_bounds__(256) void rope_kernel(float* X, const float* CS, int64_t L, int H, int D,
                                                    int64_t sin_off, int64_t row_stride, int64_t col_off) {
@@ -983,7 +1014,11 @@ int rmsnorm_launch(anima_ctx* c, const float* x, const float* w, float* y, int64
   if (rows < 0 || cols < 1) return fail(c, ANIMA_E_ARG, "anima_rmsnorm: rows=%lld cols=%d", (long long)rows, cols);
   if (rows == 0) return ANIMA_OK;
   Launch lc(c, "rmsnorm", 0.0, (double)rows * cols * 8);
-  hipLaunchKernelGGL(rmsnorm_kernel, dim3((unsigned)((rows + 3) / 4)), dim3(256), 0, c->stream, x, w, y, rows, cols, eps);
+  const dim3 grid((unsigned)((rows + 3) / 4));
+  if (cols <= 256) hipLaunchKernelGGL(rmsnorm_reg_kernel<4>, grid, dim3(256), 0, c->stream, x, w, y, rows, cols, eps);
+  else if (cols <= 1024) hipLaunchKernelGGL(rmsnorm_reg_kernel<16>, grid, dim3(256), 0, c->stream, x, w, y, rows, cols, eps);
+  else if (cols <= 2048) hipLaunchKernelGGL(rmsnorm_reg_kernel<32>, grid, dim3(256), 0, c->stream, x, w, y, rows, cols, eps);
+  else hipLaunchKernelGGL(rmsnorm_kernel, grid, dim3(256), 0, c->stream, x, w, y, rows, cols, eps);
   return lc.end();
 }
 

@@ -793,6 +793,30 @@ def test_grouped_bf16_gemv(ctx):
         ctx.linear_grouped_bf16(G, 9, N, K, dx, K, K, dw, N * K, db, 0, dy, N, N)  # M > 8
 
 
+@pytest.mark.parametrize("G,N,K", [(9, 2050, 256), (3, 6145, 512), (70, 300, 72), (1, 16384, 264), (84, 6144, 256)])
+def test_short_row_gemv(ctx, G, N, K):
+    """One row against many short weight rows (several outputs per lane group): bit-exact against the general GEMV,
+    which the same product takes as the first of two rows."""
+    case(f"short-row GEMV G={G} N={N} K={K}")
+    m = amd()
+    x = orc.randn(G + N + K, 2 * G * K).reshape(2, G * K)
+    wb = (orc.randn(N + K, G * N * K).view(np.uint32) >> 16).astype(np.uint16)  # (truncated: any bf16 values do)
+    bias = orc.randn(5, N).astype(np.float32)
+    dx, dw, db, one, two = ctx.upload(x), ctx.upload(wb), ctx.upload(bias), ctx.empty((G, N)), ctx.empty((G, 2, N))
+    ctx.linear_grouped_bf16(G, 1, N, K, dx, G * K, K, dw, N * K, db, 0, one, N, N)
+    ctx.linear_grouped_bf16(G, 2, N, K, dx, G * K, K, dw, N * K, db, 0, two, N, 2 * N)
+    assert np.array_equal(one.numpy(), two.numpy()[:, 0])
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 3), (5, 100), (43, 1024), (6, 1030), (1, 2048), (3, 2049)])
+def test_rmsnorm_bit_exact(ctx, rows, cols):
+    """Rows held in registers (64 x 4, 16 or 32 columns) and longer ones."""
+    x, w = orc.randn(rows + cols, rows * cols).reshape(rows, cols), (1 + 0.1 * orc.randn(7, cols)).astype(np.float32)
+    dy = ctx.empty((rows, cols))
+    ctx.rmsnorm(ctx.upload(x), ctx.upload(w), dy, rows, cols)
+    assert np.array_equal(dy.numpy(), orc.rmsnorm(x, w, cols))
+
+
 def test_linear_rejects_bad_arguments(ctx):
     case("linear argument validation")
     m = amd()
