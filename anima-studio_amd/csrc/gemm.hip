@@ -2240,63 +2240,109 @@ __global__ __launch_bounds__(128 * KG) void gemm_bf16_s3_kernel(F32WArgs a) {
 // workgroup (2 x 2 waves, each 32 rows x 64 columns) computes a 64 x 128 tile with both operand
 // tiles staged through double-buffered LDS, 32 k per step (x split once per workgroup as it is
 // stored; each x row read from memory once per 128 columns and each weight row once per 64 rows,
-// where the register-operand kernel reads them once per wave).  LDS rows of 40 bf16 (80 bytes)
+// where the register-operand kernel reads them once per wave).  A step's loads are issued AHEAD
+// steps before it is stored.  KG = 2: a second group of four waves takes the second half of k in LDS
+// buffers of its own and the halves are added at the end: with a workgroup per CU or less, one wave
+// per SIMD runs its reads, products, splits and stores in turn (the text encoder's
+// linears at 512 tokens, from weights that no cache of the CUs holds any more: 4096 x 1024 24.0 -> 18.9
+// us, 3072 x 1024 23.1 -> 17.2; at 43 tokens 8 to 10 us, most of it a launch and first loads).  LDS rows of 40 bf16 (80 bytes)
 // give conflict-free 16-byte fragment reads.  Epilogue and C^T layout of gemm_bf16_s3_kernel.
 constexpr int B3L_ROW = 40;
-__global__ __launch_bounds__(256) void gemm_bf16_s3_lds_kernel(F32WArgs a) {
-  __shared__ __attribute__((aligned(16))) bf16 xs[2][3][64 * B3L_ROW];
-  __shared__ __attribute__((aligned(16))) bf16 wsm[2][128 * B3L_ROW];
-  const int t = threadIdx.x, wave = t >> 6, lane = t & 63, lq = lane & 31, hf = lane >> 5;
+template <int KG, int AHEAD>
+__global__ __launch_bounds__(256 * KG) void gemm_bf16_s3_lds_kernel(F32WArgs a) {
+  constexpr int XS = 3 * 64 * B3L_ROW, WS = 128 * B3L_ROW, BUF = XS + WS;  // a step's x planes and weights
+  __shared__ __attribute__((aligned(16))) bf16 smem[KG * 2 * BUF];
+  const int kg = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, t = threadIdx.x & 255;
+  const int wave = t >> 6, lane = t & 63, lq = lane & 31, hf = lane >> 5;
   const int wm = wave & 1, wn = wave >> 1;
   const int mb = blockIdx.y * 64, nb = blockIdx.x * 128;
-  // loader roles: x row t/4, k (t%4)*8 .. +7; weight row t/2, k (t%2)*16 .. +15 (rows past M / N
-  // clamped to row 0: they only reach outputs that are not stored)
-  const int xr_row = t >> 2, xk = (t & 3) * 8, wr_row = t >> 1, wk = (t & 1) * 16;
+  bf16* const buf = smem + kg * 2 * BUF;
+  // loader roles: x row t/4, k 4 (t%4) .. + 3 and 16 + 4 (t%4) .. + 3; weight rows t/4 and 64 + t/4, k
+  // 8 (t%4) .. + 7 (four lanes take 64 contiguous bytes; rows past M / N clamped to row 0: they only
+  // reach outputs that are not stored)
+  const int lr = t >> 2, lc = t & 3;
   // blockIdx.z: k-slice z of a split product (x + z x_gs, w + z w_gs, partial output out + z out_gs)
   const int z = blockIdx.z;
   const int64_t ldw = a.ldw ? a.ldw : a.K;
-  const float* xsrc = a.x + z * a.x_gs + (int64_t)(mb + xr_row < a.M ? mb + xr_row : 0) * a.ldx + xk;
-  const uint16_t* wsrc = (const uint16_t*)a.w + z * a.w_gs + (int64_t)(nb + wr_row < a.N ? nb + wr_row : 0) * ldw + wk;
-  float4 xv0, xv1;
-  uint4 wv0, wv1;
-  auto load = [&](int k0) {
-    xv0 = *(const float4*)(xsrc + k0);
-    xv1 = *(const float4*)(xsrc + k0 + 4);
-    wv0 = *(const uint4*)(wsrc + k0);
-    wv1 = *(const uint4*)(wsrc + k0 + 8);
-  };
-  auto store = [&](int st) {
-    bf16x8 sp[3];
-    split3(xv0, xv1, sp);
+  const int nch = a.K / 32 / KG, kg0 = kg * nch * 32;  // steps and first k of this k-group
+  const float* xsrc = a.x + z * a.x_gs + (int64_t)(mb + lr < a.M ? mb + lr : 0) * a.ldx + 4 * lc + kg0;
+  const uint16_t* wsrc[2];
 #pragma unroll
-    for (int p = 0; p < 3; p++) *(bf16x8*)(&xs[st][p][xr_row * B3L_ROW + xk]) = sp[p];
-    *(uint4*)(&wsm[st][wr_row * B3L_ROW + wk]) = wv0;
-    *(uint4*)(&wsm[st][wr_row * B3L_ROW + wk + 8]) = wv1;
+  for (int i = 0; i < 2; i++) {
+    const int n = nb + 64 * i + lr;
+    wsrc[i] = (const uint16_t*)a.w + z * a.w_gs + (int64_t)(n < a.N ? n : 0) * ldw + 8 * lc + kg0;
+  }
+  struct Step {
+    float4 x[2];
+    uint4 w[2];
+  } sl[AHEAD];  // slot d: the next step d, d + AHEAD, ... (nch % AHEAD == 0)
+  auto load = [&](int kc, Step& v) __attribute__((always_inline)) {  // (past the last step: that one again, unused)
+    const int k0 = 32 * min(kc, nch - 1);
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+      v.x[i] = *(const float4*)(xsrc + k0 + 16 * i);
+      v.w[i] = *(const uint4*)(wsrc[i] + k0);
+    }
+  };
+  auto store = [&](int st, const Step& v) __attribute__((always_inline)) {
+    bf16x8 sp[3];
+    split3(v.x[0], v.x[1], sp);
+#pragma unroll
+    for (int p = 0; p < 3; p++) {
+      bf16* d = buf + st * BUF + (p * 64 + lr) * B3L_ROW + 4 * lc;
+      *(bf16x4*)d = bf16x4{sp[p][0], sp[p][1], sp[p][2], sp[p][3]};
+      *(bf16x4*)(d + 16) = bf16x4{sp[p][4], sp[p][5], sp[p][6], sp[p][7]};
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) *(uint4*)(buf + st * BUF + XS + (64 * i + lr) * B3L_ROW + 8 * lc) = v.w[i];
   };
   f32x16 acc[2] = {f32x16{}, f32x16{}};
-  const int nch = a.K / 32;
-  load(0);
-  store(0);
-  __syncthreads();
-  for (int kc = 0; kc < nch; kc++) {
-    const int st = kc & 1;
-    if (kc + 1 < nch) load(32 * (kc + 1));
+  auto products = [&](int st) __attribute__((always_inline)) {
 #pragma unroll
     for (int s = 0; s < 2; s++) {
       const int ko = 16 * s + 8 * hf;
       bf16x8 fw[2], fx[3];
 #pragma unroll
-      for (int u = 0; u < 2; u++) fw[u] = *(const bf16x8*)(&wsm[st][(wn * 64 + 32 * u + lq) * B3L_ROW + ko]);
+      for (int u = 0; u < 2; u++) fw[u] = *(const bf16x8*)(buf + st * BUF + XS + (wn * 64 + 32 * u + lq) * B3L_ROW + ko);
 #pragma unroll
-      for (int p = 0; p < 3; p++) fx[p] = *(const bf16x8*)(&xs[st][p][(wm * 32 + lq) * B3L_ROW + ko]);
+      for (int p = 0; p < 3; p++) fx[p] = *(const bf16x8*)(buf + st * BUF + (p * 64 + wm * 32 + lq) * B3L_ROW + ko);
       // smallest terms first: l, m, h
 #pragma unroll
       for (int p = 2; p >= 0; p--)
 #pragma unroll
         for (int u = 0; u < 2; u++) acc[u] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fw[u], fx[p], acc[u], 0, 0, 0);
     }
-    if (kc + 1 < nch) store(st ^ 1);
+  };
+#pragma unroll
+  for (int d = 0; d < AHEAD; d++) load(d, sl[d]);
+  store(0, sl[0]);
+  load(AHEAD, sl[0]);
+  __syncthreads();
+  for (int k0 = 0; k0 < nch; k0 += AHEAD)
+#pragma unroll
+    for (int d = 0; d < AHEAD; d++) {  // step k0 + d from buffer (k0 + d) % 2; the next one is stored beside it
+      const int st = AHEAD % 2 ? k0 & 1 : d & 1;
+      products(st);
+      store(st ^ 1, sl[(d + 1) % AHEAD]);
+      load(k0 + d + 1 + AHEAD, sl[(d + 1) % AHEAD]);
+      __syncthreads();
+    }
+  if constexpr (KG == 2) {  // the second k-group's sums, [quad][thread]
+    f32x4* part = (f32x4*)smem;
+    if (kg)
+#pragma unroll
+      for (int q = 0; q < 8; q++) {
+        const f32x16& v = acc[q >> 2];
+        part[q * 256 + t] = f32x4{v[4 * (q & 3)], v[4 * (q & 3) + 1], v[4 * (q & 3) + 2], v[4 * (q & 3) + 3]};
+      }
     __syncthreads();
+    if (kg) return;
+#pragma unroll
+    for (int q = 0; q < 8; q++) {
+      const f32x4 v = part[q * 256 + t];
+#pragma unroll
+      for (int e = 0; e < 4; e++) acc[q >> 2][4 * (q & 3) + e] += v[e];
+    }
   }
   const int m = mb + wm * 32 + lq;
   if (m >= a.M) return;
@@ -2333,22 +2379,37 @@ __global__ __launch_bounds__(256) void gemm_bf16_s3_lds_kernel(F32WArgs a) {
 }
 
 // The epilogue of a split-k product: out = epilogue(alpha * sum_z P[z] + bias + add) with the act
-// and store / residual / gated forms of the linear epilogues, one element per thread.
-__global__ __launch_bounds__(256) void splitk_epilogue_kernel(const float* P, int ks, F32WArgs a) {
-  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, n_el = (int64_t)a.M * a.N;
-  if (i >= n_el) return;
-  const int64_t m = i / a.N;
-  const int n = (int)(i - m * a.N);
-  float acc = P[i];
-  for (int z = 1; z < ks; z++) acc = acc + P[z * n_el + i];
-  float v = acc * a.alpha;
-  if (a.bias) v = v + a.bias[n];
-  if (a.add) v = v + a.add[m * a.ld_add + n];
-  v = apply_act(v, a.act);
+// and store / residual / gated forms of the linear epilogues, four columns per thread (N % 4 == 0,
+// 16-byte rows: what the split products need), every slice's load issued before the sums.
+template <int KS>
+__global__ __launch_bounds__(256) void splitk_epilogue_kernel(const float* P, F32WArgs a) {
+  const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x, nq = a.N >> 2;
+  if (i >= a.M * nq) return;
+  const int64_t plane = (int64_t)a.M * a.N, m = i / nq;
+  const int n = 4 * (int)(i - m * nq);
+  f32x4 p[KS];
+#pragma unroll
+  for (int z = 0; z < KS; z++) p[z] = *(const f32x4*)(P + z * plane + 4 * i);
   float* c = a.out + m * a.ldc + n;
-  if (a.epi == ANIMA_EPI_STORE) *c = v;
-  else if (a.epi == ANIMA_EPI_RESID) *c = *c + v;
-  else *c = __builtin_fmaf(a.gate[a.gate_off + n], v, *c);
+  f32x4 o = {};
+  if (a.epi != ANIMA_EPI_STORE) o = *(const f32x4*)c;
+  f32x4 v = p[0];
+#pragma unroll
+  for (int z = 1; z < KS; z++) v = v + p[z];
+  v = v * a.alpha;
+  if (a.bias) v = v + *(const f32x4*)(a.bias + n);
+  if (a.add) v = v + *(const f32x4*)(a.add + m * a.ld_add + n);
+  if (a.act != ANIMA_ACT_NONE)
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = apply_act(v[e], a.act);
+  if (a.epi == ANIMA_EPI_RESID) {
+    v = o + v;
+  } else if (a.epi == ANIMA_EPI_GATED) {
+    const f32x4 g = *(const f32x4*)(a.gate + a.gate_off + n);
+#pragma unroll
+    for (int e = 0; e < 4; e++) v[e] = __builtin_fmaf(g[e], v[e], o[e]);
+  }
+  *(f32x4*)c = v;
 }
 
 // Per-token int8 rows back to fp32, x[m][k] = q[m][k] * s[m] (one 4-byte group per thread;
@@ -2572,6 +2633,25 @@ static void gemm_i8_launch(anima_ctx* c, const GemmArgs& g, int tile, bool w4) {
 #undef GT_EPI
 }
 
+// gemm_bf16_s3_lds_kernel over ks k-slices.  Two k-groups per workgroup where the grid gives a CU one
+// workgroup at most (larger grids overlap several).
+static void s3_lds_launch(anima_ctx* c, const F32WArgs& f, int ks) {
+  const dim3 grid((f.N + 127) / 128, (f.M + 63) / 64, ks);
+  const bool two = (int64_t)grid.x * grid.y * ks <= c->num_cus && f.K % 64 == 0;
+  const int nch = f.K / 32 / (two ? 2 : 1);
+#define S3L(KG, A) hipLaunchKernelGGL((gemm_bf16_s3_lds_kernel<KG, A>), grid, dim3(256 * KG), 0, c->stream, f)
+  if (two) {
+    if (nch % 4 == 0) S3L(2, 4);
+    else if (nch % 2 == 0) S3L(2, 2);
+    else S3L(2, 1);
+  } else {
+    if (nch % 4 == 0) S3L(1, 4);
+    else if (nch % 2 == 0) S3L(1, 2);
+    else S3L(1, 1);
+  }
+#undef S3L
+}
+
 // G products of M <= 8 rows with bf16 weights.  One row and rows of at most 512 weights, for enough
 // outputs to fill the chip with several per lane group, take the kernel that keeps more rows in flight.
 static void gemv_launch(anima_ctx* c, const F32WArgs& f, int G) {
@@ -2715,7 +2795,7 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
       Launch L(c, "gemm.bf16s3", 2.0 * M * N * K, 0.0);
       const int64_t ltiles = (int64_t)((N + 127) / 128) * ((M + 63) / 64);
       if (ltiles >= 128 && (M + 63) / 64 <= 65535) {  // wide grids: LDS-staged tiles
-        hipLaunchKernelGGL(gemm_bf16_s3_lds_kernel, dim3((N + 127) / 128, (unsigned)((M + 63) / 64)), dim3(256), 0, c->stream, f);
+        s3_lds_launch(c, f, 1);
         return L.end();
       }
       // small grids over long rows: k-slices of the LDS kernel into partial outputs, then one pass
@@ -2739,11 +2819,11 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
         g.x_gs = K / ks;
         g.w_gs = K / ks;
         g.out_gs = (int64_t)M * N;
-        hipLaunchKernelGGL(gemm_bf16_s3_lds_kernel, dim3((N + 127) / 128, (unsigned)((M + 63) / 64), ks), dim3(256), 0,
-                           c->stream, g);
-        const int64_t n_el = (int64_t)M * N;
-        hipLaunchKernelGGL(splitk_epilogue_kernel, dim3((unsigned)((n_el + 255) / 256)), dim3(256), 0, c->stream,
-                           (const float*)tmp, ks, f);
+        s3_lds_launch(c, g, ks);
+        const dim3 eg((unsigned)((M * N / 4 + 255) / 256));
+        if (ks == 2) hipLaunchKernelGGL(splitk_epilogue_kernel<2>, eg, dim3(256), 0, c->stream, (const float*)tmp, f);
+        else if (ks == 4) hipLaunchKernelGGL(splitk_epilogue_kernel<4>, eg, dim3(256), 0, c->stream, (const float*)tmp, f);
+        else hipLaunchKernelGGL(splitk_epilogue_kernel<8>, eg, dim3(256), 0, c->stream, (const float*)tmp, f);
         anima_free(c, tmp);
         return L.end();
       }
