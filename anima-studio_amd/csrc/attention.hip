@@ -1127,43 +1127,48 @@ __global__ __launch_bounds__(512, 1) void attn_flash_w8(FlashArgs a) {
 constexpr int KSP32 = HD + 4;  // floats
 constexpr int VSP32 = BK + 4;
 
+// A workgroup is 64 queries: two waves of 32, and a second pair of waves that takes the odd key blocks
+// (in LDS tiles of its own), merged at the end.  Bound by the fp32 matrix cores (64 cycles an
+// instruction); 128 queries with every wave on all keys left half the chip idle at 1024 tokens and
+// waited for each block's loads, here a block ahead in registers: 512 x 512 image (1024 tokens, 16
+// heads) 215 -> 105 us.
+constexpr int BQ32 = 64;
+static_assert(BQ32 == BK, "a causal tile's last block is its diagonal, so no lane meets a block of masked keys only");
+
 template <bool NORM, bool ROPE>
-__global__ __launch_bounds__(256) void attn_flash_fp32(FlashArgs a) {
-  __shared__ __attribute__((aligned(16))) float Ks[BK * KSP32];
-  __shared__ __attribute__((aligned(16))) float Vs[HD * VSP32];
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+__global__ __launch_bounds__(256, 1) void attn_flash_fp32(FlashArgs a) {
+  __shared__ __attribute__((aligned(16))) float Ks2[2][BK * KSP32];
+  __shared__ __attribute__((aligned(16))) float Vs2[2][HD * VSP32];
+  const int tid = threadIdx.x & 127, wave = tid >> 6, lane = tid & 63;
+  const int kgrp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 7);  // key blocks kgrp, kgrp + 2, ...
+  float* const Ks = Ks2[kgrp];
+  float* const Vs = Vs2[kgrp];
   const int lq = lane & 31, hf = lane >> 5;
   const int id = xcd_remap(blockIdx.x, gridDim.x);
   const int bh = id / a.n_qt, qt = id - bh * a.n_qt;
   const int b = bh / a.H, h = bh - b * a.H, hk = h / a.group;
-  const int qi = qt * BQ + wave * 32 + lq;
+  const int qi = qt * BQ32 + wave * 32 + lq;
   const int Lk = a.kv_len[b];
   // causal: as in attn_flash_bf16 (lim: this lane's key limit; mlim: the workgroup's smallest)
   const int lim = a.causal ? min(Lk, qi + 1) : Lk;
-  const int mlim = a.causal ? min(Lk, qt * BQ + 1) : Lk;
-  const int nkb = a.causal ? min((Lk + BK - 1) / BK, (qt * BQ + BQ + BK - 1) / BK) : (Lk + BK - 1) / BK;
+  const int mlim = a.causal ? min(Lk, qt * BQ32 + 1) : Lk;
+  const int nkb = a.causal ? min((Lk + BK - 1) / BK, qt + 1) : (Lk + BK - 1) / BK;
 
-  // lane keeps Q[qi][2ks + hf] for ks = 0..63 (K-group g of a 32x32x2 MFMA = dim parity)
+  // k-step 4 g + e of the scores: dim 8 g + e in lane half 0, 8 g + 4 + e in half 1, so that a lane reads
+  // its K values four steps at a time; lane keeps Q[qi][8 g + 4 hf + e] as qv[4 g + e]
   float qv[64];
   {
     float x[64];
     load_q<NORM, ROPE>(a, b, h, qi, hf, x);
-    // x holds dims 16ks8 + 8hf + j; redistribute across the lane pair so that lane (q, g)
-    // holds the dims of parity g.  Lane hf has dims {16k + 8hf + j}; exchange with lane^32.
+    // x holds dims 16 k8 + 8 hf + j
 #pragma unroll
     for (int k8 = 0; k8 < 8; k8++)
 #pragma unroll
-      for (int j = 0; j < 8; j++) {
-        const float mine = x[8 * k8 + j];
-        const float other = __shfl_xor(mine, 32);
-        // dim of `mine` = 16k8 + 8hf + j, of `other` = 16k8 + 8(1-hf) + j
-        const float lo = hf ? other : mine;  // dim 16k8 + j
-        const float hi = hf ? mine : other;   // dim 16k8 + 8 + j
-        // keep dims with parity hf: d = 2ks + hf
-        if ((j & 1) == hf) {
-          qv[(16 * k8 + j) >> 1] = lo;
-          qv[(16 * k8 + 8 + j) >> 1] = hi;
-        }
+      for (int e = 0; e < 4; e++) {
+        const float lo = x[8 * k8 + e], hi = x[8 * k8 + 4 + e];
+        const float other = __shfl_xor(hf ? lo : hi, 32);  // half 0's dim 16 k8 + 4 + e, half 1's 16 k8 + 8 + e
+        qv[8 * k8 + e] = hf ? other : lo;
+        qv[8 * k8 + 4 + e] = hf ? hi : other;
       }
   }
 
@@ -1174,27 +1179,41 @@ __global__ __launch_bounds__(256) void attn_flash_fp32(FlashArgs a) {
   for (int i = 0; i < 4; i++) o[i] = (f32x16){};
   float m = -INFINITY, l = 0.0f;
 
-  for (int kb = 0; kb < nkb; kb++) {
-    // K tile 64 x 128 floats: thread -> row t/4, 32 floats; V^T tile 128 x 64: row t/2, 32 floats
-    {
-      const float4* ks = (const float4*)(kg + ((int64_t)kb * BK + (tid >> 2)) * HD + 32 * (tid & 3));
-      float4* kd = (float4*)(Ks + (tid >> 2) * KSP32 + 32 * (tid & 3));
-      const float4* vsrc = (const float4*)(vg + (int64_t)(tid >> 1) * a.Lkp + kb * BK + 32 * (tid & 1));
-      float4* vd = (float4*)(Vs + (tid >> 1) * VSP32 + 32 * (tid & 1));
+  // K tile 64 x 128 floats, V^T tile 128 x 64: 16 + 16 pieces of 4 floats per thread, consecutive threads
+  // consecutive pieces
+  f32x4 kr[16], vr[16];
+  auto fetch = [&](int kb) __attribute__((always_inline)) {
+    const int kc = min(kb, nkb - 1);
 #pragma unroll
-      for (int i = 0; i < 8; i++) {
-        kd[i] = ks[i];
-        vd[i] = vsrc[i];
-      }
+    for (int i = 0; i < 16; i++) {
+      const int u = 128 * i + tid;
+      kr[i] = *(const f32x4*)(kg + (int64_t)kc * BK * HD + 4 * u);
+      vr[i] = *(const f32x4*)(vg + (int64_t)(u >> 4) * a.Lkp + kc * BK + 4 * (u & 15));
+    }
+  };
+  fetch(kgrp);
+  for (int kb0 = 0; kb0 < nkb; kb0 += 2) {
+    const int kb = kb0 + kgrp;
+    if (kb0) __syncthreads();  // every wave is done with the previous blocks' tiles
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const int u = 128 * i + tid;
+      *(f32x4*)(Ks + (u >> 5) * KSP32 + 4 * (u & 31)) = kr[i];
+      *(f32x4*)(Vs + (u >> 4) * VSP32 + 4 * (u & 15)) = vr[i];
     }
     __syncthreads();
+    fetch(kb + 2);
+    if (kb >= nkb) continue;  // (the odd blocks' waves at an odd count; they meet no barrier in the rest)
     f32x16 s0 = {}, s1 = {};
-#pragma unroll 16
-    for (int ks = 0; ks < 64; ks++) {
-      const float k0 = Ks[lq * KSP32 + 2 * ks + hf];
-      const float k1 = Ks[(32 + lq) * KSP32 + 2 * ks + hf];
-      s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(k0, qv[ks], s0, 0, 0, 0);
-      s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(k1, qv[ks], s1, 0, 0, 0);
+    const float* kp = Ks + lq * KSP32 + 4 * hf;
+#pragma unroll
+    for (int g = 0; g < 16; g++) {
+      const f32x4 k0 = *(const f32x4*)(kp + 8 * g), k1 = *(const f32x4*)(kp + 32 * KSP32 + 8 * g);
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        s0 = __builtin_amdgcn_mfma_f32_32x32x2f32(k0[e], qv[4 * g + e], s0, 0, 0, 0);
+        s1 = __builtin_amdgcn_mfma_f32_32x32x2f32(k1[e], qv[4 * g + e], s1, 0, 0, 0);
+      }
     }
     if ((kb + 1) * BK > mlim) {
 #pragma unroll
@@ -1235,10 +1254,33 @@ __global__ __launch_bounds__(256) void attn_flash_fp32(FlashArgs a) {
         o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 + key], s1[r], o[dt], 0, 0, 0);
       }
     }
-    __syncthreads();
   }
 
   l += __shfl_xor(l, 32);
+  // the second pair's outputs, [quad][thread], maximum and sum through LDS
+  __syncthreads();
+  f32x4* const part = (f32x4*)&Ks2[0][0];
+  float* const ml = &Vs2[0][0];
+  static_assert(16 * 128 * 16 <= sizeof(Ks2) && 2 * 128 * 4 <= sizeof(Vs2), "the merge fits the tiles");
+  if (kgrp) {
+#pragma unroll
+    for (int i = 0; i < 16; i++)
+      part[i * 128 + tid] = f32x4{o[i >> 2][4 * (i & 3)], o[i >> 2][4 * (i & 3) + 1], o[i >> 2][4 * (i & 3) + 2], o[i >> 2][4 * (i & 3) + 3]};
+    ml[tid] = m;
+    ml[128 + tid] = l;
+  }
+  __syncthreads();
+  if (kgrp) return;
+  if (nkb > 1) {
+    const float m1 = ml[tid], mn = fmaxf(m, m1), f0 = __builtin_amdgcn_exp2f(m - mn), f1 = __builtin_amdgcn_exp2f(m1 - mn);
+    l = l * f0 + ml[128 + tid] * f1;
+#pragma unroll
+    for (int i = 0; i < 16; i++) {
+      const f32x4 v = part[i * 128 + tid];
+#pragma unroll
+      for (int e = 0; e < 4; e++) o[i >> 2][4 * (i & 3) + e] = o[i >> 2][4 * (i & 3) + e] * f0 + v[e] * f1;
+    }
+  }
   if (qi < a.Lq) {
     const float inv = 1.0f / l;
     float* dst = a.o + (int64_t)b * a.o_bs + (int64_t)qi * a.ldo + h * a.D + 4 * hf;
@@ -1432,7 +1474,7 @@ int attention_launch_ws(anima_ctx* c, const anima_attn_desc* d, void* scratch) {
   // (the Q copies of a workgroup use 32-bit offsets: 256 rows of ldq fp32)
   const bool w8 = bf && !d->causal && d->D == HD && (int64_t)((d->Lq + W8_BQ - 1) / W8_BQ) * d->H * d->B >= c->num_cus &&
                   (int64_t)W8_BQ * (d->q_prep ? d->H * HD / 2 : d->ldq) * 4 < (1LL << 31);
-  f.n_qt = w8 ? (d->Lq + W8_BQ - 1) / W8_BQ : (d->Lq + BQ - 1) / BQ;
+  f.n_qt = w8 ? (d->Lq + W8_BQ - 1) / W8_BQ : bf ? (d->Lq + BQ - 1) / BQ : (d->Lq + BQ32 - 1) / BQ32;
   for (int b = 0; b < MAXB; b++) f.kv_len[b] = b < d->B ? kv_len[b] : 1;
   f.causal = d->causal ? 1 : 0;
   f.D = d->D;
