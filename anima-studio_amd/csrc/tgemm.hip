@@ -1,12 +1,12 @@
 // Tiled bf16-MFMA GEMM for fp32 activations, and what the VAE decoder builds on it:
-//   * conv3x3 (pad 1) of an NHWC image as an implicit GEMM, with the 2x nearest upsample of the
-//     input fused into the operand loads and the residual add into the epilogue (the "conv3" loader
-//     of app/gpu/gemm.js:56-80, dispatched by ops.conv3x3 / conv3x3Into, app/gpu/ops.js:95-109);
+//   * conv3x3 (pad 1) of an NHWC image, with the 2x nearest upsample of the input and the residual add
+//     fused (the "conv3" loader of app/gpu/gemm.js:56-80, dispatched by ops.conv3x3 / conv3x3Into,
+//     app/gpu/ops.js:95-109): by rows, on spatial tiles, or as an implicit GEMM;
 //   * the Wan channel norm y = x / max(||x||, 1e-12) * sqrt(C) * gamma (+ SiLU) of
 //     app/gpu/kernels.js:62-89 (mode 1), in the shader's reduction order;
-//   * attention for head dims other than 128 (the LLM adapter's 64, the VAE's single 384-dim head),
-//     on the reference's chunked path (app/gpu/ops.js:177-207): scores for a chunk of query rows, a
-//     row softmax (optionally causal), then P.V.
+//   * attention for head dims other than 128: 384 (the VAE's single head) fused, others on the
+//     reference's chunked path (app/gpu/ops.js:177-207): scores for a chunk of query rows, a row
+//     softmax (optionally causal), then P.V.
 //
 // The GEMM: C[m][n] = alpha * sum_k A[m][k] B[n][k] (* rs[m]) (+ bias[n]) (act), stored or added
 // to C.  One workgroup = 4 waves = a 128 x 128 output tile, each wave 64 x 64 (2 x 2 tiles of
