@@ -2915,15 +2915,15 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
   // (a LoRA epilogue always runs on the int8 grid: the in-GEMM unpack leaves it no registers)
   if (w4 && tile >= 0 && (c->w4_path == ANIMA_W4_GRID_SCRATCH || (tile == GT_256 && lora))) {
     rc = w4_grid_scratch(c, W, g, &grid8);
-    // no memory for the grid: only the 256x256 kernel's callers ever depended on it
-    if (rc && !(rc == ANIMA_E_OOM && tile != GT_256)) {
+    if (rc && rc != ANIMA_E_OOM) {
       if (tmp) anima_free(c, tmp);
       return rc;
     }
     if (!rc) w4k = false;
+    else (void)hipGetLastError();  // no memory for the grid: the codes are unpacked inside the GEMM
     rc = ANIMA_OK;
   }
-  if (w4k && tile != GT_256) tile = -1;
+  if (w4k && (tile != GT_256 || lora)) tile = -1;
   // otherwise the LoRA product is an add term (the split-bf16 kernel, one product per rank block
   // over its columns' rows of the B planes)
   void* ldelta = nullptr;

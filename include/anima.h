@@ -489,8 +489,8 @@ int anima_weight_unpack_w4(anima_ctx* ctx, const anima_weight* w4, int8_t* grid)
  *   ANIMA_W4_GRID_SCRATCH (default): one pass writes the weight's int8 grid (anima_weight_unpack_w4
  *     semantics) into a pooled scratch buffer of N * K bytes, released after the call; the int8
  *     GEMM reads it.  The weight stays packed in memory; the nibble work runs once per call
- *     instead of once per row tile.  (A product that does not take the 256 x 256 tile unpacks
- *     inside its GEMM if there is no memory for the grid.)
+ *     instead of once per row tile.  (anima_linear unpacks inside its GEMM if there is no
+ *     memory for the grid.)
  *   ANIMA_W4_IN_GEMM: every workgroup unpacks its B tiles inside the GEMM main loop (no scratch). */
 #define ANIMA_W4_GRID_SCRATCH 0
 #define ANIMA_W4_IN_GEMM 1
