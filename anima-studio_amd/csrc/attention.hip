@@ -1127,32 +1127,35 @@ __global__ __launch_bounds__(512, 1) void attn_flash_w8(FlashArgs a) {
 constexpr int KSP32 = HD + 4;  // floats
 constexpr int VSP32 = BK + 4;
 
-// A workgroup is 64 queries: two waves of 32, and a second pair of waves that takes the odd key blocks
-// (in LDS tiles of its own), merged at the end.  Bound by the fp32 matrix cores (64 cycles an
-// instruction); 128 queries with every wave on all keys left half the chip idle at 1024 tokens and
-// waited for each block's loads, here a block ahead in registers: 512 x 512 image (1024 tokens, 16
-// heads) 215 -> 105 us.
-constexpr int BQ32 = 64;
-static_assert(BQ32 == BK, "a causal tile's last block is its diagonal, so no lane meets a block of masked keys only");
+// Bound by the fp32 matrix cores (64 cycles an instruction).  KG = 2: a workgroup is 64 queries: two waves of
+// 32, and a second pair of waves that takes the odd key blocks (in LDS tiles of its own), merged at the end,
+// the next block's loads in registers meanwhile.  For grids that leave CUs idle (1024 tokens, 16 heads: 223 ->
+// 110 us against 128 queries with every wave on all keys) and causal masks.  KG = 1: 128 queries, every wave on
+// all keys, two workgroups per CU, which cover each other's loads and prologues: 4096 tokens x 64 / 1024 / 4096 keys, 16
+// heads, 46 / 289 / 1069 us (KG = 2: 92 / 365 / 1290).
+template <int KG>
+constexpr int BQ32 = 128 / KG;
+static_assert(BQ32<2> == BK, "a causal tile's last block is its diagonal, so no lane meets a block of masked keys only");
 
-template <bool NORM, bool ROPE>
-__global__ __launch_bounds__(256, 1) void attn_flash_fp32(FlashArgs a) {
-  __shared__ __attribute__((aligned(16))) float Ks2[2][BK * KSP32];
-  __shared__ __attribute__((aligned(16))) float Vs2[2][HD * VSP32];
-  const int tid = threadIdx.x & 127, wave = tid >> 6, lane = tid & 63;
-  const int kgrp = __builtin_amdgcn_readfirstlane(threadIdx.x >> 7);  // key blocks kgrp, kgrp + 2, ...
+template <bool NORM, bool ROPE, int KG>
+__global__ __launch_bounds__(256, 3 - KG) void attn_flash_fp32(FlashArgs a) {
+  constexpr int NT = 256 / KG, NP = 2048 / NT;  // threads of a key group; pieces of 4 floats per thread and tile
+  __shared__ __attribute__((aligned(16))) float Ks2[KG][BK * KSP32];
+  __shared__ __attribute__((aligned(16))) float Vs2[KG][HD * VSP32];
+  const int tid = threadIdx.x & (NT - 1), wave = tid >> 6, lane = tid & 63;
+  const int kgrp = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / NT) : 0;  // key blocks kgrp, kgrp + KG, ...
   float* const Ks = Ks2[kgrp];
   float* const Vs = Vs2[kgrp];
   const int lq = lane & 31, hf = lane >> 5;
   const int id = xcd_remap(blockIdx.x, gridDim.x);
   const int bh = id / a.n_qt, qt = id - bh * a.n_qt;
   const int b = bh / a.H, h = bh - b * a.H, hk = h / a.group;
-  const int qi = qt * BQ32 + wave * 32 + lq;
+  const int qi = qt * BQ32<KG> + wave * 32 + lq;
   const int Lk = a.kv_len[b];
   // causal: as in attn_flash_bf16 (lim: this lane's key limit; mlim: the workgroup's smallest)
   const int lim = a.causal ? min(Lk, qi + 1) : Lk;
-  const int mlim = a.causal ? min(Lk, qt * BQ32 + 1) : Lk;
-  const int nkb = a.causal ? min((Lk + BK - 1) / BK, qt + 1) : (Lk + BK - 1) / BK;
+  const int mlim = a.causal ? min(Lk, qt * BQ32<KG> + 1) : Lk;
+  const int nkb = a.causal ? min((Lk + BK - 1) / BK, (qt + 1) * (BQ32<KG> / BK)) : (Lk + BK - 1) / BK;
 
   // k-step 4 g + e of the scores: dim 8 g + e in lane half 0, 8 g + 4 + e in half 1, so that a lane reads
   // its K values four steps at a time; lane keeps Q[qi][8 g + 4 hf + e] as qv[4 g + e]
@@ -1179,30 +1182,31 @@ __global__ __launch_bounds__(256, 1) void attn_flash_fp32(FlashArgs a) {
   for (int i = 0; i < 4; i++) o[i] = (f32x16){};
   float m = -INFINITY, l = 0.0f;
 
-  // K tile 64 x 128 floats, V^T tile 128 x 64: 16 + 16 pieces of 4 floats per thread, consecutive threads
+  // K tile 64 x 128 floats, V^T tile 128 x 64: NP + NP pieces of 4 floats per thread, consecutive threads
   // consecutive pieces
-  f32x4 kr[16], vr[16];
+  f32x4 kr[NP], vr[NP];
   auto fetch = [&](int kb) __attribute__((always_inline)) {
     const int kc = min(kb, nkb - 1);
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      const int u = 128 * i + tid;
+    for (int i = 0; i < NP; i++) {
+      const int u = NT * i + tid;
       kr[i] = *(const f32x4*)(kg + (int64_t)kc * BK * HD + 4 * u);
       vr[i] = *(const f32x4*)(vg + (int64_t)(u >> 4) * a.Lkp + kc * BK + 4 * (u & 15));
     }
   };
-  fetch(kgrp);
-  for (int kb0 = 0; kb0 < nkb; kb0 += 2) {
+  if (KG > 1) fetch(kgrp);
+  for (int kb0 = 0; kb0 < nkb; kb0 += KG) {
     const int kb = kb0 + kgrp;
+    if (KG == 1) fetch(kb);  // (a block ahead it spills: two workgroups per CU cover the loads)
     if (kb0) __syncthreads();  // every wave is done with the previous blocks' tiles
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      const int u = 128 * i + tid;
+    for (int i = 0; i < NP; i++) {
+      const int u = NT * i + tid;
       *(f32x4*)(Ks + (u >> 5) * KSP32 + 4 * (u & 31)) = kr[i];
       *(f32x4*)(Vs + (u >> 4) * VSP32 + 4 * (u & 15)) = vr[i];
     }
     __syncthreads();
-    fetch(kb + 2);
+    if (KG > 1) fetch(kb + KG);
     if (kb >= nkb) continue;  // (the odd blocks' waves at an odd count; they meet no barrier in the rest)
     f32x16 s0 = {}, s1 = {};
     const float* kp = Ks + lq * KSP32 + 4 * hf;
@@ -1237,48 +1241,68 @@ __global__ __launch_bounds__(256, 1) void attn_flash_fp32(FlashArgs a) {
 #pragma unroll
       for (int i = 0; i < 4; i++) o[i] *= alpha;
     }
+    float bl = KG == 1 ? 0.0f : l;  // (KG = 1: the block's sum by itself)
 #pragma unroll
     for (int r = 0; r < 16; r++) {
       s0[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s0[r], a.c, -m));
       s1[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s1[r], a.c, -m));
-      l += s0[r] + s1[r];
+      bl += s0[r] + s1[r];
     }
+    l = KG == 1 ? l + bl : bl;
     // k-step (tile t, register r): keys 32t + 8(r/4) + 4g + r%4 for k-group g
-#pragma unroll
-    for (int r = 0; r < 16; r++) {
-      const int key = 8 * (r >> 2) + 4 * hf + (r & 3);
+    if constexpr (KG == 1) {
+      // the block's products by themselves, then added: chains of one per block across blocks (error against 64 bits
+      // at 1024 / 4096 keys 4.3e-7 / 4.7e-7, in one chain 7.1e-7 / 1.26e-6; KG = 2 has no registers for it)
 #pragma unroll
       for (int dt = 0; dt < 4; dt++) {
         const float* vrow = Vs + (32 * dt + lq) * VSP32;
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[key], s0[r], o[dt], 0, 0, 0);
-        o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 + key], s1[r], o[dt], 0, 0, 0);
+        f32x16 p = {};
+#pragma unroll
+        for (int r = 0; r < 16; r++) {
+          const int key = 8 * (r >> 2) + 4 * hf + (r & 3);
+          p = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[key], s0[r], p, 0, 0, 0);
+          p = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 + key], s1[r], p, 0, 0, 0);
+        }
+        o[dt] += p;
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; r++) {
+        const int key = 8 * (r >> 2) + 4 * hf + (r & 3);
+#pragma unroll
+        for (int dt = 0; dt < 4; dt++) {
+          const float* vrow = Vs + (32 * dt + lq) * VSP32;
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[key], s0[r], o[dt], 0, 0, 0);
+          o[dt] = __builtin_amdgcn_mfma_f32_32x32x2f32(vrow[32 + key], s1[r], o[dt], 0, 0, 0);
+        }
       }
     }
   }
 
   l += __shfl_xor(l, 32);
-  // the second pair's outputs, [quad][thread], maximum and sum through LDS
-  __syncthreads();
-  f32x4* const part = (f32x4*)&Ks2[0][0];
-  float* const ml = &Vs2[0][0];
-  static_assert(16 * 128 * 16 <= sizeof(Ks2) && 2 * 128 * 4 <= sizeof(Vs2), "the merge fits the tiles");
-  if (kgrp) {
+  if constexpr (KG == 2) {  // the second pair's outputs, [quad][thread], maximum and sum through LDS
+    __syncthreads();
+    f32x4* const part = (f32x4*)&Ks2[0][0];
+    float* const ml = &Vs2[0][0];
+    static_assert(16 * 128 * 16 <= sizeof(Ks2) && 2 * 128 * 4 <= sizeof(Vs2), "the merge fits the tiles");
+    if (kgrp) {
 #pragma unroll
-    for (int i = 0; i < 16; i++)
-      part[i * 128 + tid] = f32x4{o[i >> 2][4 * (i & 3)], o[i >> 2][4 * (i & 3) + 1], o[i >> 2][4 * (i & 3) + 2], o[i >> 2][4 * (i & 3) + 3]};
-    ml[tid] = m;
-    ml[128 + tid] = l;
-  }
-  __syncthreads();
-  if (kgrp) return;
-  if (nkb > 1) {
-    const float m1 = ml[tid], mn = fmaxf(m, m1), f0 = __builtin_amdgcn_exp2f(m - mn), f1 = __builtin_amdgcn_exp2f(m1 - mn);
-    l = l * f0 + ml[128 + tid] * f1;
+      for (int i = 0; i < 16; i++)
+        part[i * 128 + tid] = f32x4{o[i >> 2][4 * (i & 3)], o[i >> 2][4 * (i & 3) + 1], o[i >> 2][4 * (i & 3) + 2], o[i >> 2][4 * (i & 3) + 3]};
+      ml[tid] = m;
+      ml[128 + tid] = l;
+    }
+    __syncthreads();
+    if (kgrp) return;
+    if (nkb > 1) {
+      const float m1 = ml[tid], mn = fmaxf(m, m1), f0 = __builtin_amdgcn_exp2f(m - mn), f1 = __builtin_amdgcn_exp2f(m1 - mn);
+      l = l * f0 + ml[128 + tid] * f1;
 #pragma unroll
-    for (int i = 0; i < 16; i++) {
-      const f32x4 v = part[i * 128 + tid];
+      for (int i = 0; i < 16; i++) {
+        const f32x4 v = part[i * 128 + tid];
 #pragma unroll
-      for (int e = 0; e < 4; e++) o[i >> 2][4 * (i & 3) + e] = o[i >> 2][4 * (i & 3) + e] * f0 + v[e] * f1;
+        for (int e = 0; e < 4; e++) o[i >> 2][4 * (i & 3) + e] = o[i >> 2][4 * (i & 3) + e] * f0 + v[e] * f1;
+      }
     }
   }
   if (qi < a.Lq) {
@@ -1353,6 +1377,20 @@ static int attention_check(anima_ctx* c, const anima_attn_desc* d, int (&kv_len)
     if (!al16(d->rope_cs)) return fail(c, ANIMA_E_ARG, "anima_attention: rope_cs must be 16-byte aligned");
   }
   return ANIMA_OK;
+}
+
+// Key groups of the fp32 kernel, by the measured time of both forms (us; n blocks of 64 keys): 128-query
+// workgroups run two to a CU in 16.4 n + 16, a single one in 9 n + 12; a 64-query workgroup with two key groups takes
+// 10.4 ceil(n / 2) + 14, one to a CU.  Under a causal mask of several blocks the second form balances better
+// (4096 tokens, 16 heads: 860 us, the first 1056).
+static int fp32_key_groups(int num_cus, const anima_attn_desc* d) {
+  const int64_t bh = (int64_t)d->B * d->H, n = d->causal ? std::min((d->Lk + BK - 1) / BK, (d->Lq + BK - 1) / BK) : (d->Lk + BK - 1) / BK;
+  if (d->causal && n > 1) return 2;
+  const int64_t w1 = (bh * ((d->Lq + BQ32<1> - 1) / BQ32<1>) + num_cus - 1) / num_cus,
+                w2 = (bh * ((d->Lq + BQ32<2> - 1) / BQ32<2>) + num_cus - 1) / num_cus;
+  const double t1 = (double)(w1 / 2) * (16.4 * n + 16) + (double)(w1 % 2) * (9.0 * n + 12),
+               t2 = (double)w2 * (10.4 * ((n + 1) / 2) + 14);
+  return t1 <= t2 ? 1 : 2;
 }
 
 // The K/V prep of one attention call into dst ([K plane][V^T plane], each B Hkv Lkp HD elements).
@@ -1474,7 +1512,8 @@ int attention_launch_ws(anima_ctx* c, const anima_attn_desc* d, void* scratch) {
   // (the Q copies of a workgroup use 32-bit offsets: 256 rows of ldq fp32)
   const bool w8 = bf && !d->causal && d->D == HD && (int64_t)((d->Lq + W8_BQ - 1) / W8_BQ) * d->H * d->B >= c->num_cus &&
                   (int64_t)W8_BQ * (d->q_prep ? d->H * HD / 2 : d->ldq) * 4 < (1LL << 31);
-  f.n_qt = w8 ? (d->Lq + W8_BQ - 1) / W8_BQ : bf ? (d->Lq + BQ - 1) / BQ : (d->Lq + BQ32 - 1) / BQ32;
+  const int kg32 = bf ? 0 : fp32_key_groups(c->num_cus, d);
+  f.n_qt = w8 ? (d->Lq + W8_BQ - 1) / W8_BQ : bf ? (d->Lq + BQ - 1) / BQ : kg32 == 1 ? (d->Lq + BQ32<1> - 1) / BQ32<1> : (d->Lq + BQ32<2> - 1) / BQ32<2>;
   for (int b = 0; b < MAXB; b++) f.kv_len[b] = b < d->B ? kv_len[b] : 1;
   f.causal = d->causal ? 1 : 0;
   f.D = d->D;
@@ -1483,9 +1522,13 @@ int attention_launch_ws(anima_ctx* c, const anima_attn_desc* d, void* scratch) {
   double flops = 0;
   for (int b = 0; b < d->B; b++) flops += 4.0 * d->Lq * (double)kv_len[b] * d->D * d->H;
   const int blocks = f.n_qt * d->H * d->B;
-  Launch L(c, w8 ? "attn.flash_bf16" : bf ? "attn.flash_bf16_4w" : "attn.flash_fp32", flops, 0.0);
+  Launch L(c, w8 ? "attn.flash_bf16" : bf ? "attn.flash_bf16_4w" : kg32 == 1 ? "attn.flash_fp32" : "attn.flash_fp32_2g", flops, 0.0);
   const bool qn = d->q_norm != nullptr;
-#define FLASH(K, N, R) hipLaunchKernelGGL((K<N, R>), dim3(blocks), dim3(256), 0, c->stream, f)
+#define FLASH(N, R)                                                                                                    \
+  do {                                                                                                                \
+    if (kg32 == 2) hipLaunchKernelGGL((attn_flash_fp32<N, R, 2>), dim3(blocks), dim3(256), 0, c->stream, f);          \
+    else hipLaunchKernelGGL((attn_flash_fp32<N, R, 1>), dim3(blocks), dim3(256), 0, c->stream, f);                    \
+  } while (0)
 #define FLASHB(T, N, R) hipLaunchKernelGGL((attn_flash_bf16<T, N, R>), dim3(blocks), dim3(256), 0, c->stream, f)
   if (f.qp && w8) {
     hipLaunchKernelGGL((attn_flash_w8<false, false, true>), dim3(blocks), dim3(512), 0, c->stream, f);
@@ -1504,10 +1547,10 @@ int attention_launch_ws(anima_ctx* c, const anima_attn_desc* d, void* scratch) {
     else if (rope) FLASHB(FLASH_KB, false, true);
     else FLASHB(FLASH_KB, false, false);
   } else {
-    if (qn && rope) FLASH(attn_flash_fp32, true, true);
-    else if (qn) FLASH(attn_flash_fp32, true, false);
-    else if (rope) FLASH(attn_flash_fp32, false, true);
-    else FLASH(attn_flash_fp32, false, false);
+    if (qn && rope) FLASH(true, true);
+    else if (qn) FLASH(true, false);
+    else if (rope) FLASH(false, true);
+    else FLASH(false, false);
   }
 #undef FLASH
 #undef FLASHB

@@ -361,6 +361,41 @@ def test_head_dim_64_flash_path(ctx, precision):
                 assert r <= (1e-5 if precision == "fp32" else 1e-2)
 
 
+@pytest.mark.parametrize("B,Lq,Lk,H,group,causal,kv_len,form", [
+    (1, 4096, 64, 16, 1, 0, None, "attn.flash_fp32"), (1, 64, 60, 2, 1, 1, None, "attn.flash_fp32"),
+    (4, 300, 200, 16, 2, 0, [200, 64, 1, 130], "attn.flash_fp32"), (2, 1300, 512, 8, 1, 0, [449, 512], "attn.flash_fp32"),
+    (1, 129, 200, 2, 1, 0, None, "attn.flash_fp32_2g"), (2, 65, 320, 4, 2, 0, [320, 63], "attn.flash_fp32_2g"),
+    (1, 192, 192, 2, 1, 1, None, "attn.flash_fp32_2g"), (3, 130, 77, 2, 1, 1, [77, 70, 5], "attn.flash_fp32_2g")])
+def test_fp32_forms(ctx, B, Lq, Lk, H, group, causal, kv_len, form):
+    """Both forms of the fp32 kernel (128-query workgroups on all keys; 64-query ones with two key groups) where the
+    rule takes them, with remainders in queries and keys, masks and grouped heads, against float64; few keys under
+    many queries run the first form (the second leaves half of each workgroup idle there)."""
+    case(f"fp32 attention {form} B={B} Lq={Lq} Lk={Lk} H={H} causal={causal}")
+    m = amd()
+    D, Hk = HD, H // group
+    rng = np.random.default_rng(Lq + Lk)
+    q, k, v = (rng.standard_normal((B, n, h * D)).astype(np.float32) for n, h in ((Lq, H), (Lk, Hk), (Lk, Hk)))
+    dq, dk, dv, do = ctx.upload(q), ctx.upload(k), ctx.upload(v), ctx.empty((B, Lq, H * D))
+    ctx.profile(True)
+    ctx.profile_reset()
+    ctx.attention(q=dq, k=dk, v=dv, o=do, B=B, Lq=Lq, Lk=Lk, H=H, D=D, ldq=H * D, ldk=Hk * D, ldv=Hk * D, group=group,
+                  kv_len=kv_len, causal=causal, precision=m.PREC_FP32)
+    names = [r["name"] for r in ctx.profile_report()]
+    ctx.profile(False)
+    assert form in names, names
+    got = do.numpy()
+    for b in range(B):
+        n = kv_len[b] if kv_len else Lk
+        for h in (0, H - 1):
+            s = q[b, :, h * D:(h + 1) * D].astype(np.float64) @ k[b, :n, h // group * D:(h // group + 1) * D].astype(np.float64).T / np.sqrt(D)
+            if causal:
+                s = np.where(np.arange(n)[None] <= np.arange(Lq)[:, None], s, -np.inf)
+            w = np.exp(s - s.max(-1, keepdims=True))
+            ref = w @ v[b, :n, h // group * D:(h // group + 1) * D] / w.sum(-1, keepdims=True)
+            r, _ = report(f"b={b} h={h} vs float64", got[b, :, h * D:(h + 1) * D], ref)
+            assert r <= 1e-5
+
+
 # ------------------------------------------------------------------ ragged shapes, GQA, strides
 
 @pytest.mark.parametrize("precision", ["bf16", "fp32"])
