@@ -1235,17 +1235,19 @@ __global__ __launch_bounds__(256, 3 - KG) void attn_flash_fp32(FlashArgs a) {
     const bool need = bmc > m + RESCALE_SLACK;
     if (__builtin_amdgcn_ballot_w64(need)) {
       const float mn = need ? ceilf(bmc) : m;
-      const float alpha = __builtin_amdgcn_exp2f(m - mn);
+      const float alpha = need ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;  // (m may be -inf still)
       m = mn;
       l *= alpha;
 #pragma unroll
       for (int i = 0; i < 4; i++) o[i] *= alpha;
     }
+    // no finite score so far: weights of zero (as they are beside the finite scores of other key blocks)
+    const float mf = m == -INFINITY ? 0.0f : m;
     float bl = KG == 1 ? 0.0f : l;  // (KG = 1: the block's sum by itself)
 #pragma unroll
     for (int r = 0; r < 16; r++) {
-      s0[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s0[r], a.c, -m));
-      s1[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s1[r], a.c, -m));
+      s0[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s0[r], a.c, -mf));
+      s1[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s1[r], a.c, -mf));
       bl += s0[r] + s1[r];
     }
     l = KG == 1 ? l + bl : bl;

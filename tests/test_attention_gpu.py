@@ -396,6 +396,36 @@ def test_fp32_forms(ctx, B, Lq, Lk, H, group, causal, kv_len, form):
             assert r <= 1e-5
 
 
+@pytest.mark.parametrize("B,H,Lq,Lk,blocks,form", [
+    (1, 2, 70, 200, [1], "attn.flash_fp32_2g"), (1, 2, 70, 300, [0, 2], "attn.flash_fp32_2g"),
+    (1, 2, 70, 300, [1, 3], "attn.flash_fp32_2g"), (4, 16, 300, 200, [0, 1], "attn.flash_fp32")])
+def test_fp32_key_blocks_of_infinite_scores(ctx, B, H, Lq, Lk, blocks, form):
+    """Whole 64-key blocks whose scores overflow to -inf weigh nothing, whichever key group takes them: the result is
+    the attention over the other keys."""
+    case(f"fp32 attention, key blocks {blocks} of {Lk} keys at -inf")
+    m = amd()
+    rng = np.random.default_rng(Lk + len(blocks))
+    q = (1e20 * rng.uniform(0.5, 1.5, (B, Lq, H * HD))).astype(np.float32)
+    k = (1e-20 * rng.standard_normal((B, Lk, H * HD))).astype(np.float32)
+    v = rng.standard_normal((B, Lk, H * HD)).astype(np.float32)
+    masked = np.isin(np.arange(Lk) // 64, blocks)
+    k[:, masked] = -1e20
+    dq, dk, dv, do = ctx.upload(q), ctx.upload(k), ctx.upload(v), ctx.empty((B, Lq, H * HD))
+    ctx.profile(True)
+    ctx.profile_reset()
+    ctx.attention(q=dq, k=dk, v=dv, o=do, B=B, Lq=Lq, Lk=Lk, H=H, D=HD, ldq=H * HD, ldk=H * HD, ldv=H * HD, precision=m.PREC_FP32)
+    names = [r["name"] for r in ctx.profile_report()]
+    ctx.profile(False)
+    assert form in names, names
+    got = do.numpy()
+    for h in range(H):
+        c = slice(h * HD, (h + 1) * HD)
+        s = q[0, :, c].astype(np.float64) @ k[0, ~masked, c].astype(np.float64).T / np.sqrt(HD)
+        w = np.exp(s - s.max(-1, keepdims=True))
+        r, _ = report(f"h={h} vs float64", got[0, :, c], w @ v[0, ~masked, c] / w.sum(-1, keepdims=True))
+        assert r <= 1e-5
+
+
 # ------------------------------------------------------------------ ragged shapes, GQA, strides
 
 @pytest.mark.parametrize("precision", ["bf16", "fp32"])
