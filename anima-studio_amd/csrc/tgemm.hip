@@ -1230,7 +1230,7 @@ __global__ __launch_bounds__(512, 2) void attn384_kernel(FaArgs a, int nitem) {
       for (int r = 1; r < 16; r++) mx = fmaxf(mx, y[r]);
       mx = fmaxf(mx, __shfl_xor(mx, 32));
       if (__any(mx > m)) {  // (rare once the first blocks are done)
-        const float mn = fmaxf(m, mx), al = __builtin_amdgcn_exp2f(m - mn);
+        const float mn = fmaxf(m, mx), al = mx > m ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;  // (m may be -inf still)
         m = mn;
         l = l * al;
 #pragma unroll
@@ -1239,13 +1239,15 @@ __global__ __launch_bounds__(512, 2) void attn384_kernel(FaArgs a, int nitem) {
       // the next block's scores beside this block's weights (after the last block: of the last again, unused)
       S = f32x16{};
       scores(S);
+      // no finite score so far: weights of zero (as they are beside the finite scores of other key blocks)
+      const float mf = m == -INFINITY ? 0.0f : m;
       bf16x8 ph[2], pl[2];
 #pragma unroll
       for (int s2 = 0; s2 < 2; s2++) {
         float e[8];
 #pragma unroll
         for (int r = 0; r < 8; r++) {
-          e[r] = __builtin_amdgcn_exp2f(y[8 * s2 + r] - m);
+          e[r] = __builtin_amdgcn_exp2f(y[8 * s2 + r] - mf);
           l += e[r];
         }
         fa_split<SPLIT>(e, ph[s2], pl[s2]);

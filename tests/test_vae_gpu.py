@@ -154,6 +154,36 @@ def test_chunked_attention_matches_float64(case, precision):
             assert r <= (2e-5 if precision == "fp32" else 1e-2)
 
 
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+@pytest.mark.parametrize("lo,hi", [(0, 32), (0, 320), (96, 544), (960, 1000)])
+def test_attention_384_key_blocks_of_infinite_scores(lo, hi, precision):
+    """384-dim heads: 32-key blocks, and whole key splits, whose scores overflow to -inf weigh nothing (values exact in
+    bf16, so that no rest of the split overflows the other way)."""
+    m = amd()
+    print(f"[case] 384-dim attention, keys {lo} .. {hi - 1} of 1000 at -inf, {precision}", flush=True)
+    rng = np.random.default_rng(lo + hi)
+    bf = lambda x: (x.astype(np.float32).view(np.uint32) & 0xFFFF0000).view(np.float32)
+    q = bf(rng.uniform(1.0, 2.0, (40, 384))) * np.float32(2.0**66)
+    k = bf(rng.standard_normal((1000, 384))) * np.float32(2.0**-66)
+    v = rng.standard_normal((1000, 384)).astype(np.float32)
+    k[lo:hi] = -(2.0**66)
+    with m.Context() as ctx:
+        dq, dk, dv, do = ctx.upload(q), ctx.upload(k), ctx.upload(v), ctx.empty((40, 384))
+        ctx.profile(True)
+        ctx.attention(q=dq, k=dk, v=dv, o=do, B=1, Lq=40, Lk=1000, H=1, D=384, ldq=384, ldk=384, ldv=384,
+                      precision=m.PREC_FP32 if precision == "fp32" else m.PREC_BF16)
+        names = [r["name"] for r in ctx.profile_report()]
+        assert "attn.384" in names, names
+        got = do.numpy()
+        for b in (dq, dk, dv, do):
+            b.release()
+    ok = (np.arange(1000) < lo) | (np.arange(1000) >= hi)
+    s = q.astype(np.float64) @ k[ok].astype(np.float64).T / math.sqrt(384)
+    w = np.exp(s - s.max(-1, keepdims=True))
+    r, _ = report(f"384-dim attention {precision} vs float64", got, w @ v[ok] / w.sum(-1, keepdims=True))
+    assert r <= (2e-5 if precision == "fp32" else 1e-2)
+
+
 def _attn_rows_f64(q, k, v, rows, D, causal, n=None):
     """float64 softmax(q k^T / sqrt(D)) v for the given query rows of one head (keys < n; with
     causal, keys <= row as well)."""
