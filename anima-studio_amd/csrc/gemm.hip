@@ -2567,6 +2567,15 @@ static bool al(const void* p, int b) { return ((uintptr_t)p & (b - 1)) == 0; }
 enum { GT_256, GT_256x128, GT_128, GT_64x128, GT_32x64, GT_COUNT };
 enum { GT_PLAIN, GT_LORA, GT_OPERANDS, GT_OPERANDS_LORA };  // epilogues
 
+// Profiler names: the tile (-1: gemm_i8_kernel), W4 codes decoded in the GEMM, attention operands.
+static const char* gemm_i8_name(int tile, bool w4, bool kv) {
+  static const char* const names[2][2][GT_COUNT + 1] = {
+      {{"gemm.i8.general", "gemm.i8.256x256", "gemm.i8.256x128", "gemm.i8.128x128", "gemm.i8.64x128", "gemm.i8.32x64"},
+       {"gemm.i8_qkv.general", "gemm.i8_qkv.256x256", "gemm.i8_qkv.256x128", "gemm.i8_qkv.128x128", "gemm.i8_qkv.64x128", ""}},
+      {{"gemm.w4a8.general", "gemm.w4a8.256x256", "", "", "", ""}, {"", "gemm.w4a8_qkv.256x256", "", "", "", ""}}};
+  return names[w4][kv][tile + 1];
+}
+
 static int gemm_i8_cols(int tile) { return tile == GT_256 ? 256 : tile == GT_32x64 ? 64 : 128; }
 
 // Measured time of one output tile per CU, microseconds: base (launch, first loads, epilogue) +
@@ -2907,13 +2916,14 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
   // aligned output rows, scales, bias and gate (gemm_i8_kernel takes what is left).
   const bool vec = N % 4 == 0 && g.ldc % 4 == 0 && al(g.out, 16) && al(g.sw, 16) && (!g.bias || al(g.bias, 16)) &&
                    (g.epi != ANIMA_EPI_GATED || al(g.gate + g.gate_off, 16)) && (!g.add || (al(g.add, 16) && g.ld_add % 4 == 0));
-  int tile = vec ? gemm_i8_choose(c, M, N, K, lora ? GT_LORA : GT_PLAIN) : -1;
-  // the LoRA product in the epilogue: a tile's columns lie in one rank block
-  const bool lepi = lora && tile >= 0 && d->lora_cols % gemm_i8_cols(tile) == 0;
+  // a 256x256 tile for every CU: of the two kernels that decode W4 codes, the 256x256 one takes these products (its
+  // decode runs beside the matrix cores: 4096 x 6144 x 2048 103 us, gemm_i8_kernel 163) and the other the rest
+  const int64_t tiles256 = (int64_t)((N + 255) / 256) * ((M + 255) / 256);
+  const bool big = vec && tiles256 >= c->num_cus && tiles256 <= 0x7fffffff;
   void* grid8 = nullptr;
   bool w4k = w4;  // the GEMM unpacks W4 codes itself
-  // (a LoRA epilogue always runs on the int8 grid: the in-GEMM unpack leaves it no registers)
-  if (w4 && tile >= 0 && (c->w4_path == ANIMA_W4_GRID_SCRATCH || (tile == GT_256 && lora))) {
+  // (the LoRA epilogue of a tile runs on the int8 grid: the in-GEMM unpack leaves it no registers)
+  if (w4 && vec && (c->w4_path == ANIMA_W4_GRID_SCRATCH || (big && lora))) {
     rc = w4_grid_scratch(c, W, g, &grid8);
     if (rc && rc != ANIMA_E_OOM) {
       if (tmp) anima_free(c, tmp);
@@ -2923,11 +2933,13 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
     else (void)hipGetLastError();  // no memory for the grid: the codes are unpacked inside the GEMM
     rc = ANIMA_OK;
   }
-  if (w4k && (tile != GT_256 || lora)) tile = -1;
+  const int tile = !vec ? -1 : !w4k ? gemm_i8_choose(c, M, N, K, lora ? GT_LORA : GT_PLAIN) : big && !lora ? (int)GT_256 : -1;
+  // the LoRA product in the epilogue: a tile's columns lie in one rank block
+  const bool lepi = lora && tile >= 0 && d->lora_cols % gemm_i8_cols(tile) == 0;
   // otherwise the LoRA product is an add term (the split-bf16 kernel, one product per rank block
   // over its columns' rows of the B planes)
   void* ldelta = nullptr;
-  if (lora && !(lepi && tile >= 0)) {
+  if (lora && !lepi) {
     rc = anima_alloc(c, (size_t)M * N * 4, &ldelta);
     if (rc) {
       if (grid8) anima_free(c, grid8);
@@ -2952,12 +2964,12 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
     g.lr = 0;
   }
   if (!rc) {
-    Launch L(c, w4k ? "gemm.w4a8" : "gemm.i8", 2.0 * M * N * K, 0.0);
+    Launch L(c, gemm_i8_name(tile, w4k, false), 2.0 * M * N * K, 0.0);
     if (tile >= 0) {
       gemm_i8_launch(c, g, tile, w4k);
     } else {
       dim3 grid((N + GBN - 1) / GBN, (unsigned)((M + GBM - 1) / GBM));
-      if (w4) hipLaunchKernelGGL(gemm_i8_kernel<true>, grid, dim3(256), 0, c->stream, g);
+      if (w4k) hipLaunchKernelGGL(gemm_i8_kernel<true>, grid, dim3(256), 0, c->stream, g);
       else hipLaunchKernelGGL(gemm_i8_kernel<false>, grid, dim3(256), 0, c->stream, g);
     }
     rc = L.end();
@@ -3078,9 +3090,9 @@ int linear_qkv_launch(anima_ctx* c, const anima_linear_desc* d, const anima_qkv_
     w4 = false;
   }
   {
-    Launch L(c, w4 ? "gemm.w4a8_qkv" : "gemm.i8_qkv", 2.0 * M * N * K, 0.0);
     // (a 256-column tile holds two whole heads, a 128-column tile one; in-GEMM W4 decode: 256x256 only)
     const int tile = w4 ? (int)GT_256 : gemm_i8_choose(c, M, N, K, lora ? GT_OPERANDS_LORA : GT_OPERANDS);
+    Launch L(c, gemm_i8_name(tile, w4, true), 2.0 * M * N * K, 0.0);
     // (the prepared-Q epilogue is an instance of its own: its code raises the register pressure of
     // the main loop it shares the kernel with)
     if (lora && g.qp) gemm_i8_launch_t<ANIMA_EPI_STORE, true, true, true>(c, g, tile, w4);

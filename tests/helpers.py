@@ -38,3 +38,14 @@ def report(name, got, ref):
     r, m = rel_l2(got, ref), max_abs(got, ref)
     print(f"{name}: rel L2 {r:.3e}  max|d| {m:.3e}", flush=True)
     return r, m
+
+
+def ran(ctx, call):
+    """The profiler names of what `call` launched."""
+    ctx.sync()
+    ctx.profile(True)
+    ctx.profile_reset()
+    call()
+    names = {r["name"] for r in ctx.profile_report()}
+    ctx.profile(False)
+    return names

@@ -13,7 +13,7 @@ import numpy as np
 import pytest
 
 import oracle as orc
-from helpers import amd, rel_l2, report
+from helpers import amd, ran, rel_l2, report
 
 pytestmark = pytest.mark.gpu
 
@@ -361,6 +361,42 @@ def test_int8_tile_sizes(ctx, M, N, K, kind):
     ref = (q.astype(np.float64) @ w.astype(np.float64).T).astype(np.int32)  # exact: |sums| < 2^53
     assert np.array_equal(acc.numpy(), ref)
     assert np.array_equal(out.numpy(), c0 + (ref.astype(np.float32) * sx[:, None]) * s)
+
+
+@pytest.mark.parametrize("M,N,K,lora,kernel", [
+    (4096, 6144, 128, 0, "gemm.w4a8.256x256"), (2300, 8196, 192, 0, "gemm.w4a8.256x256"),
+    (1000, 2048, 128, 0, "gemm.w4a8.general"), (4096, 6146, 64, 0, "gemm.w4a8.general"),
+    (4100, 4100, 128, 32, "gemm.i8."), (1000, 2048, 128, 32, "gemm.w4a8.general")])
+def test_w4_in_gemm_kernels(ctx, w4_path, M, N, K, lora, kernel):
+    """W4 codes decoded inside the GEMM: products with a 256x256 tile for every CU run the 256x256 kernel (whatever tile
+    the same product takes on int8 weights), the rest the general one; with a LoRA the first run on the scratch grid
+    with the term in the epilogue.  Exact sums; bits of the same product on the int8 grid."""
+    case(f"W4 in the GEMM M={M} N={N} K={K} lora={lora}")
+    m = amd()
+    codes, srel, sw = w4_weight(K, N, K)
+    grid = orc.w4_decode(codes, srel, FIXED_LUT, N, K)
+    W = m.weight(m.W_W4, N, K, ctx.upload(codes), scale=ctx.upload(sw), srel=ctx.upload(srel), codebook=ctx.upload(FIXED_LUT))
+    W8 = m.weight(m.W_I8, N, K, ctx.upload(grid), scale=ctx.upload(sw))
+    rng = np.random.default_rng(M + N)
+    q = rng.integers(-127, 128, size=(M, K), dtype=np.int8)
+    c0 = rng.standard_normal((M, N)).astype(np.float32)
+    dq, ds = ctx.upload(q), ctx.upload(rng.uniform(0.5, 1.5, M).astype(np.float32) / 127)
+    kw = {}
+    if lora:
+        planes = ctx.empty(3 * N * lora, np.uint16)
+        ctx.split3_bf16(ctx.upload((0.05 * rng.standard_normal((N, lora))).astype(np.float32)), planes, N * lora)
+        kw = dict(lora_xa=ctx.upload(rng.standard_normal((M, lora)).astype(np.float32)), ld_lora_xa=lora, lora_b=planes, lora_r=lora)
+    out, acc, out8 = ctx.upload(c0), ctx.empty((M, N), np.int32), ctx.upload(c0)
+    w4_path("in_gemm")
+    names = ran(ctx, lambda: ctx.linear(W, M, out, xq=dq, xs=ds, epilogue=m.EPI_RESID, acc_out=acc, **kw))
+    assert any(n.startswith(kernel) for n in names), names
+    assert ("gemm.f32s3" in names) == (lora > 0 and kernel == "gemm.w4a8.general"), names  # the LoRA term as an add term
+    assert np.array_equal(acc.numpy(), (q.astype(np.float32) @ grid.astype(np.float32).T).astype(np.int32))  # |sums| < 2^24
+    ctx.linear(W8, M, out8, xq=dq, xs=ds, epilogue=m.EPI_RESID, **kw)
+    if lora:
+        assert report("against the int8 grid", out.numpy(), out8.numpy())[0] <= 2e-6
+    else:
+        assert np.array_equal(out.numpy(), out8.numpy())
 
 
 @pytest.mark.parametrize("act,epi", [("gelu", 0), ("silu", 1)])
