@@ -2565,7 +2565,7 @@ static bool al(const void* p, int b) { return ((uintptr_t)p & (b - 1)) == 0; }
 // so small products take small tiles (more of them), and products of several rounds take the tile
 // whose last round is fullest.
 enum { GT_256, GT_256x128, GT_128, GT_64x128, GT_32x64, GT_COUNT };
-enum { GT_PLAIN, GT_LORA, GT_OPERANDS, GT_OPERANDS_LORA };  // epilogues
+enum { GT_STORE, GT_RESID, GT_LORA, GT_OPERANDS, GT_OPERANDS_LORA };  // epilogues
 
 // Profiler names: the tile (-1: gemm_i8_kernel), W4 codes decoded in the GEMM, attention operands.
 static const char* gemm_i8_name(int tile, bool w4, bool kv) {
@@ -2578,22 +2578,33 @@ static const char* gemm_i8_name(int tile, bool w4, bool kv) {
 
 static int gemm_i8_cols(int tile) { return tile == GT_256 ? 256 : tile == GT_32x64 ? 64 : 128; }
 
-// Measured time of one output tile per CU, microseconds: base (launch, first loads, epilogue) +
-// step * K / 2048, for each further tile per CU step * K / 2048 more.  Fitted to M = 256 .. 8192,
-// N = 2048 / 6144 / 8192, K = 2048 / 8192, at K = 2048 and M x N of 256 x 2048: 32x64 6.8 (128x128
-// 16); 1024 x 2048: 64x128 12.4 (256x256 39.5, the former 128x128 loop 38.6; K = 8192 29.8 / 97 /
-// 104); 2240 x 2048: 256x128 27.7 (43.7); 2240 x 8192: 128x128 63 (69.6); 7904 x 2048: 256x256 57.4
-// (128x128 66.7).
+// Microseconds of a product on one tile size: base (launch, first loads, the last epilogue) + for each tile per CU
+// step * K / 2048, and round for each one after the first (its epilogue).  Per epilogue: the stored output is much of a
+// short product.  Fitted to 3276 products of M = 1 .. 16384, N = 64 .. 8192, K = 64 .. 8192 (1575 with a LoRA, 900
+// with attention operands): the choice takes 1.1 / 0.4% longer than the best tile in the mean (plain / residual), 0.3%
+// the others.  The constants of one sum per tile, fitted at K >= 2048, took 12 / 8 / 9% at all K (4096 x 4096 x 64: 32x64 tiles 43 us,
+// 256x256 26).  Another tile than 256x256 has to be 4% faster where that one has a tile for every CU (it varies least
+// from run to run), and stored products of K < 512 stay there (bound by their stores: 12288 x 2048 x 128 26 us, 128x128 32).
 static int gemm_i8_choose(anima_ctx* c, int64_t M, int N, int K, int kind) {
-  static const struct { int bm, bn; float base, step; } T[GT_COUNT] = {
-      {256, 256, 18.0f, 24.0f}, {256, 128, 8.0f, 17.0f}, {128, 128, 8.5f, 9.0f}, {64, 128, 6.0f, 6.5f}, {32, 64, 3.3f, 3.5f}};
+  static const struct { int bm, bn; } T[GT_COUNT] = {{256, 256}, {256, 128}, {128, 128}, {64, 128}, {32, 64}};
+  static const struct { float base, step, round; } P[5][GT_COUNT] = {
+      {{10.5f, 19.3f, 21.3f}, {7.0f, 10.9f, 15.5f}, {6.0f, 8.2f, 4.2f}, {4.8f, 5.3f, 3.8f}, {4.1f, 1.9f, 0.8f}},    // store
+      {{15.6f, 16.3f, 27.8f}, {15.3f, 8.9f, 17.5f}, {6.2f, 7.3f, 6.3f}, {5.9f, 5.6f, 5.3f}, {3.8f, 1.9f, 1.0f}},    // residual, gate
+      {{41.5f, 21.0f, 56.2f}, {16.2f, 10.3f, 32.6f}, {12.5f, 7.4f, 12.4f}, {10.0f, 4.9f, 10.9f}, {}},               // LoRA
+      {{29.8f, 20.8f, 31.5f}, {16.5f, 13.2f, 15.8f}, {12.1f, 9.4f, 4.9f}, {7.1f, 6.1f, 2.2f}, {}},                  // operands
+      {{39.6f, 37.6f, 44.3f}, {19.8f, 11.3f, 24.6f}, {16.2f, 8.4f, 7.6f}, {7.5f, 5.5f, 4.0f}, {}}};                 // operands + LoRA
   int best = -1;
   float bt = 0.0f;
   for (int t = 0; t < GT_COUNT; t++) {
-    if (t == GT_32x64 && kind != GT_PLAIN) continue;  // (a head, or a rank block, is 128 columns wide)
-    const int64_t tiles = (N + T[t].bn - 1) / T[t].bn * ((M + T[t].bm - 1) / T[t].bm);
+    if (t == GT_32x64 && kind >= GT_LORA) continue;  // (a head, or a rank block, is 128 columns wide)
+    const int64_t tiles = (int64_t)((N + T[t].bn - 1) / T[t].bn) * ((M + T[t].bm - 1) / T[t].bm);
     if (tiles > 0x7fffffff || (t != GT_256 && K > 65536)) continue;  // (tile rows times K: 32-bit offsets)
-    const float us = T[t].base + T[t].step * (float)K / 2048.0f * (float)((tiles + c->num_cus - 1) / c->num_cus);
+    const float rounds = (float)((tiles + c->num_cus - 1) / c->num_cus);
+    float us = P[kind][t].base + P[kind][t].step * (float)K / 2048.0f * rounds + P[kind][t].round * (rounds - 1.0f);
+    if (t == GT_256 && tiles >= c->num_cus) {
+      if (kind == GT_STORE && K < 512) return GT_256;
+      us = us / 1.04f;
+    }
     if (best < 0 || us < bt) {
       best = t;
       bt = us;
@@ -2933,7 +2944,7 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
     else (void)hipGetLastError();  // no memory for the grid: the codes are unpacked inside the GEMM
     rc = ANIMA_OK;
   }
-  const int tile = !vec ? -1 : !w4k ? gemm_i8_choose(c, M, N, K, lora ? GT_LORA : GT_PLAIN) : big && !lora ? (int)GT_256 : -1;
+  const int tile = !vec ? -1 : !w4k ? gemm_i8_choose(c, M, N, K, lora ? GT_LORA : g.epi == ANIMA_EPI_STORE ? GT_STORE : GT_RESID) : big && !lora ? (int)GT_256 : -1;
   // the LoRA product in the epilogue: a tile's columns lie in one rank block
   const bool lepi = lora && tile >= 0 && d->lora_cols % gemm_i8_cols(tile) == 0;
   // otherwise the LoRA product is an add term (the split-bf16 kernel, one product per rank block

@@ -399,6 +399,23 @@ def test_w4_in_gemm_kernels(ctx, w4_path, M, N, K, lora, kernel):
         assert np.array_equal(out.numpy(), out8.numpy())
 
 
+@pytest.mark.parametrize("M,N,K,epi,lora,tile", [
+    (4096, 4096, 64, "store", 0, "256x256"), (12288, 2048, 128, "store", 0, "256x256"), (8192, 2048, 256, "resid", 0, "256x256"),
+    (4096, 4096, 192, "resid", 0, "256x256"), (4096, 4096, 1024, "store", 0, "256x256"), (4096, 4096, 192, "resid", 32, "256x256"),
+    (2304, 8192, 1024, "resid", 0, "128x128"), (2200, 2048, 2048, "resid", 0, "256x128"), (1000, 2048, 2048, "resid", 0, "64x128"),
+    (4000, 1152, 1024, "store", 32, "256x128"), (200, 2048, 2048, "store", 0, "32x64"), (1, 64, 64, "store", 0, "32x64")])
+def test_int8_tile_choice(ctx, M, N, K, epi, lora, tile):
+    """The tile an int8 product runs on: short rows leave the stores as the cost, so products with a 256x256 tile for every
+    CU stay there at any K (tiles for K of 2048 and up took up to 1.7 times as long); the exact results are the other tests'."""
+    m = amd()
+    buf = ctx.empty((M * N + 3 * (M + N) * (K + lora),))
+    ctx.zero(buf, M * N)
+    W = m.weight(m.W_I8, N, K, buf, scale=buf)
+    kw = dict(lora_xa=buf, ld_lora_xa=lora, lora_b=buf, lora_r=lora) if lora else {}
+    names = ran(ctx, lambda: ctx.linear(W, M, ctx.empty((M, N)), xq=buf, xs=buf, epilogue=m.EPI_STORE if epi == "store" else m.EPI_RESID, **kw))
+    assert names == {"gemm.i8." + tile}, names
+
+
 @pytest.mark.parametrize("act,epi", [("gelu", 0), ("silu", 1)])
 def test_256_tile_kernel_activation_epilogues(ctx, act, epi):
     """The 256x256 kernel with GELU (store) and SiLU (residual add) epilogues at M=4000, N=4100:
