@@ -2613,6 +2613,16 @@ static int gemm_i8_choose(anima_ctx* c, int64_t M, int N, int K, int kind) {
   return best;
 }
 
+// W4 products of few rows whose in-GEMM decode (gemm_i8_kernel: us by measurement, rounds of one 128-column tile per CU)
+// is shorter than the unpack pass and the product after it: one launch instead of two (1 x 2048 x 256 7.4 us, with
+// the pass 9.6; 1 x 24576 x 1024 14.5 and 25.5; 1 x 2048 x 1024 14.5 and 9.7).
+static bool w4_few_rows(anima_ctx* c, int64_t M, int N, int K) {
+  if (M > 32) return false;
+  const float rounds = (float)(((N + 127) / 128 + c->num_cus - 1) / c->num_cus);
+  const float in_gemm = (5.0f + 9.2f * (float)K / 1024.0f) * rounds + 0.2f * (float)M, pass = 3.5f + 1e-6f * (float)N * (float)K;
+  return in_gemm < (pass > 9.5f ? pass : 9.5f);
+}
+
 template <int EPI, bool KV, bool QP, bool LORA>
 static void gemm_i8_launch_t(anima_ctx* c, const GemmArgs& g, int tile, bool w4) {
   const auto tiles = [&](int bm, int bn) { return (unsigned)((int64_t)((g.N + bn - 1) / bn) * ((g.M + bm - 1) / bm)); };
@@ -2934,7 +2944,8 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
   void* grid8 = nullptr;
   bool w4k = w4;  // the GEMM unpacks W4 codes itself
   // (the LoRA epilogue of a tile runs on the int8 grid: the in-GEMM unpack leaves it no registers)
-  if (w4 && vec && (c->w4_path == ANIMA_W4_GRID_SCRATCH || (big && lora))) {
+  if (w4 && vec && (lora ? big || c->w4_path == ANIMA_W4_GRID_SCRATCH
+                         : c->w4_path == ANIMA_W4_GRID_SCRATCH && !w4_few_rows(c, M, N, K))) {
     rc = w4_grid_scratch(c, W, g, &grid8);
     if (rc && rc != ANIMA_E_OOM) {
       if (tmp) anima_free(c, tmp);

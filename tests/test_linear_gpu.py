@@ -399,6 +399,27 @@ def test_w4_in_gemm_kernels(ctx, w4_path, M, N, K, lora, kernel):
         assert np.array_equal(out.numpy(), out8.numpy())
 
 
+@pytest.mark.parametrize("M,N,K,kernel", [(1, 2048, 256, "gemm.w4a8.general"), (8, 256, 128, "gemm.w4a8.general"),
+                                          (1, 24576, 512, "gemm.w4a8.general"), (1, 2048, 1024, "gemm.i8.32x64"),
+                                          (33, 2048, 64, "gemm.i8.32x64")])
+def test_w4_few_rows(ctx, M, N, K, kernel):
+    """W4 products of few rows decode their codes in the GEMM where that is shorter than unpacking first: exact sums,
+    the store epilogue bit for bit."""
+    case(f"W4 few rows M={M} N={N} K={K}")
+    m = amd()
+    codes, srel, sw = w4_weight(K + M, N, K)
+    W = m.weight(m.W_W4, N, K, ctx.upload(codes), scale=ctx.upload(sw), srel=ctx.upload(srel), codebook=ctx.upload(FIXED_LUT))
+    rng = np.random.default_rng(M + N)
+    q = rng.integers(-127, 128, size=(M, K), dtype=np.int8)
+    sx = (rng.uniform(0.5, 1.5, M) / 127).astype(np.float32)
+    dq, ds, out, acc = ctx.upload(q), ctx.upload(sx), ctx.empty((M, N)), ctx.empty((M, N), np.int32)
+    names = ran(ctx, lambda: ctx.linear(W, M, out, xq=dq, xs=ds, acc_out=acc))
+    assert kernel in names and ("w4.unpack" in names) == (kernel != "gemm.w4a8.general"), names
+    ref = orc.gemm_i8(q, orc.w4_decode(codes, srel, FIXED_LUT, N, K))
+    assert np.array_equal(acc.numpy(), ref)
+    assert np.array_equal(out.numpy(), orc.linear_epilogue(ref, sx, sw))
+
+
 @pytest.mark.parametrize("M,N,K,epi,lora,tile", [
     (4096, 4096, 64, "store", 0, "256x256"), (12288, 2048, 128, "store", 0, "256x256"), (8192, 2048, 256, "resid", 0, "256x256"),
     (4096, 4096, 192, "resid", 0, "256x256"), (4096, 4096, 1024, "store", 0, "256x256"), (4096, 4096, 192, "resid", 32, "256x256"),
