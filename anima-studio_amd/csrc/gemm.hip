@@ -2682,10 +2682,14 @@ static void s3_lds_launch(anima_ctx* c, const F32WArgs& f, int ks) {
 #undef S3L
 }
 
-// G products of M <= 8 rows with bf16 weights.  One row and rows of at most 512 weights, for enough
-// outputs to fill the chip with several per lane group, take the kernel that keeps more rows in flight.
+// One row and rows of at most 512 weights, for enough outputs to fill the chip with several per lane group, take the
+// kernel that keeps more rows in flight; products of 8 outputs and fewer leave most of its lane groups idle (20000 of
+// one output 39 us, one wave per output 13; 13108 of 10 outputs 28 and 40).
+static bool gemv_is_short(const F32WArgs& f, int G) { return f.M == 1 && f.K <= 512 && f.N > 8 && (int64_t)G * f.N >= 16384; }
+
+// G products of M <= 8 rows with bf16 weights.
 static void gemv_launch(anima_ctx* c, const F32WArgs& f, int G) {
-  if (f.M == 1 && f.K <= 512 && (int64_t)G * f.N >= 16384) {
+  if (gemv_is_short(f, G)) {
     if (f.K <= 256) hipLaunchKernelGGL((gemv_short_kernel<32, 8>), dim3((f.N + 63) / 64, (unsigned)G), dim3(256), 0, c->stream, f);
     else hipLaunchKernelGGL((gemv_short_kernel<64, 8>), dim3((f.N + 31) / 32, (unsigned)G), dim3(256), 0, c->stream, f);
   } else {
@@ -2812,7 +2816,7 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
     F32WArgs f{d->x, ldx, W->w, W->bias, d->out, ldc, alpha, d->act, d->epilogue, d->gate, d->gate_off,
                (int)M, N, K, 0, 0, 0, 0, d->add, ld_add, f32 ? 1 : 0};
     if (!f32 && M <= GEMV_MAXM && K % 8 == 0 && ldx % 4 == 0 && al(d->x, 16) && al(W->w, 16)) {
-      Launch L(c, "gemv.bf16", 2.0 * M * N * K, 2.0 * N * K);
+      Launch L(c, gemv_is_short(f, 1) ? "gemv.bf16.short" : "gemv.bf16", 2.0 * M * N * K, 2.0 * N * K);
       gemv_launch(c, f, 1);
       return L.end();
     }
@@ -3141,7 +3145,7 @@ int linear_grouped_bf16_launch(anima_ctx* c, int G, int64_t M, int N, int K, con
     return fail(c, ANIMA_E_ARG, "anima_linear_grouped_bf16: x and w must be 16-byte aligned (ldx, x stride %% 4, w stride %% 8)");
   F32WArgs f{x, ldx, w, bias, out, ldc, 1.0f, ANIMA_ACT_NONE, ANIMA_EPI_STORE, nullptr, 0, (int)M, N, K,
              x_gs, w_gs, bias_gs, out_gs, nullptr, 0, 0};
-  Launch L(c, "gemv.bf16.grouped", 2.0 * G * M * N * K, 2.0 * G * N * K);
+  Launch L(c, gemv_is_short(f, G) ? "gemv.bf16.grouped.short" : "gemv.bf16.grouped", 2.0 * G * M * N * K, 2.0 * G * N * K);
   gemv_launch(c, f, G);
   return L.end();
 }

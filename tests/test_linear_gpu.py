@@ -867,17 +867,19 @@ def test_grouped_bf16_gemv(ctx):
         ctx.linear_grouped_bf16(G, 9, N, K, dx, K, K, dw, N * K, db, 0, dy, N, N)  # M > 8
 
 
-@pytest.mark.parametrize("G,N,K", [(9, 2050, 256), (3, 6145, 512), (70, 300, 72), (1, 16384, 264), (84, 6144, 256)])
+@pytest.mark.parametrize("G,N,K", [(9, 2050, 256), (3, 6145, 512), (70, 300, 72), (1, 16384, 264), (84, 6144, 256),
+                                   (20000, 1, 512), (2048, 8, 64), (1821, 9, 256)])
 def test_short_row_gemv(ctx, G, N, K):
-    """One row against many short weight rows (several outputs per lane group): bit-exact against the general GEMV,
-    which the same product takes as the first of two rows."""
+    """One row against many short weight rows (several outputs per lane group, from 9 outputs and 16384 in all): bit-exact
+    against the general GEMV, which the same product takes as the first of two rows."""
     case(f"short-row GEMV G={G} N={N} K={K}")
     m = amd()
     x = orc.randn(G + N + K, 2 * G * K).reshape(2, G * K)
     wb = (orc.randn(N + K, G * N * K).view(np.uint32) >> 16).astype(np.uint16)  # (truncated: any bf16 values do)
     bias = orc.randn(5, N).astype(np.float32)
     dx, dw, db, one, two = ctx.upload(x), ctx.upload(wb), ctx.upload(bias), ctx.empty((G, N)), ctx.empty((G, 2, N))
-    ctx.linear_grouped_bf16(G, 1, N, K, dx, G * K, K, dw, N * K, db, 0, one, N, N)
+    names = ran(ctx, lambda: ctx.linear_grouped_bf16(G, 1, N, K, dx, G * K, K, dw, N * K, db, 0, one, N, N))
+    assert names == {"gemv.bf16.grouped.short" if N > 8 else "gemv.bf16.grouped"}, names
     ctx.linear_grouped_bf16(G, 2, N, K, dx, G * K, K, dw, N * K, db, 0, two, N, 2 * N)
     assert np.array_equal(one.numpy(), two.numpy()[:, 0])
 
