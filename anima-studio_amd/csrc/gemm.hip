@@ -2938,8 +2938,9 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
   }
   int rc = ANIMA_OK;
   // The tiled kernels' epilogues move 16-byte column groups: they need N % 4 == 0 and 16-byte
-  // aligned output rows, scales, bias and gate (gemm_i8_kernel takes what is left).
-  const bool vec = N % 4 == 0 && g.ldc % 4 == 0 && al(g.out, 16) && al(g.sw, 16) && (!g.bias || al(g.bias, 16)) &&
+  // aligned output rows, scales, bias and gate, and 32-bit offsets into a tile's 256 rows (gemm_i8_kernel takes
+  // what is left).
+  const bool vec = K < (1 << 23) && N % 4 == 0 && g.ldc % 4 == 0 && al(g.out, 16) && al(g.sw, 16) && (!g.bias || al(g.bias, 16)) &&
                    (g.epi != ANIMA_EPI_GATED || al(g.gate + g.gate_off, 16)) && (!g.add || (al(g.add, 16) && g.ld_add % 4 == 0));
   // a 256x256 tile for every CU: of the two kernels that decode W4 codes, the 256x256 one takes these products (its
   // decode runs beside the matrix cores: 4096 x 6144 x 2048 103 us, gemm_i8_kernel 163) and the other the rest

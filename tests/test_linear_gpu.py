@@ -399,6 +399,24 @@ def test_w4_in_gemm_kernels(ctx, w4_path, M, N, K, lora, kernel):
         assert np.array_equal(out.numpy(), out8.numpy())
 
 
+def test_int8_rows_past_32_bit_offsets(ctx):
+    """Rows so long that 256 of them pass 4 GiB run the kernel with 64-bit offsets: exact sums of ones times n + 1."""
+    case("int8 product of 258 rows of 2^24")
+    m = amd()
+    M, N, K = 258, 4, 1 << 24
+    q, one = ctx.empty((M * K,), np.int8), ctx.upload(np.ones(M, np.float32))
+    ctx.fill_random(q, M * K, "u8", 1, 1, 1)
+    w = ctx.upload(np.repeat(np.arange(1, N + 1, dtype=np.int8)[:, None], K, 1))
+    W = m.weight(m.W_I8, N, K, w, scale=one)
+    out, acc = ctx.empty((M, N)), ctx.empty((M, N), np.int32)
+    names = ran(ctx, lambda: ctx.linear(W, M, out, xq=q, xs=one, acc_out=acc))
+    assert names == {"gemm.i8.general"}, names
+    assert np.array_equal(acc.numpy(), np.tile(K * np.arange(1, N + 1), (M, 1)))
+    q.release()
+    w.release()
+    ctx.trim()
+
+
 @pytest.mark.parametrize("M,N,K,kernel", [(1, 2048, 256, "gemm.w4a8.general"), (8, 256, 128, "gemm.w4a8.general"),
                                           (1, 24576, 512, "gemm.w4a8.general"), (1, 2048, 1024, "gemm.i8.32x64"),
                                           (33, 2048, 64, "gemm.i8.32x64")])
