@@ -1346,10 +1346,11 @@ static int attention384_launch(anima_ctx* c, const anima_attn_desc* d, const int
   if (a.kv_head >= (1LL << 31) || bytes > (1LL << 30) || wgs * a.splits > 0x7fffffff || bh > 65535 || Hk > 65535) return 0;
   void* ws = nullptr;
   int rc = workspace(c, (size_t)bytes, &ws);
-  if (rc) {
+  if (rc == ANIMA_E_OOM) {
     (void)hipGetLastError();
     return 0;  // (the chunked path asks for its own amount)
   }
+  if (rc) return rc;
   a.q = d->q + d->q_off;
   a.k = d->k + d->k_off;
   a.v = d->v + d->v_off;
