@@ -461,14 +461,14 @@ constexpr int CR_COLS = 30, CR_LDS = 110592, CR_WLDS = 4096;  // weights; a wave
 constexpr int CR_MAXK = CR_LDS / (9 * 2);  // input channels times BN
 
 
-__device__ __forceinline__ f32x4 cr_load(__amdgpu_buffer_rsrc_t r, int voff, int soff) {
+__device__ __forceinline__ f32x4 cr_load(__amdgpu_buffer_rsrc_t r, unsigned voff, int soff) {
   const auto v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
   return __builtin_bit_cast(f32x4, v);
 }
 // The whole offset in the vector register: with a scalar register as the offset, the compiler lets the
 // next vector instruction overwrite the data of a 16-byte store (no hazard on older chips), and first
 // components of outputs came out wrong here.
-__device__ __forceinline__ void cr_store(__amdgpu_buffer_rsrc_t r, int voff, f32x4 v) {
+__device__ __forceinline__ void cr_store(__amdgpu_buffer_rsrc_t r, unsigned voff, f32x4 v) {
   typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
   __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, v), r, voff, 0, 0);
 }
@@ -541,13 +541,14 @@ __global__ __launch_bounds__(512, 2) void conv3x3_rows_kernel(TGemmArgs p, int R
   const int n = n0 + 16 * g + 4 * lg;  // this lane's four channels
   // this lane's pixel of each tile, as read (pixel lane / 4, channels 4 (lane % 4) .. + 3 of each half of
   // the step) and as multiplied and written: columns outside the image read zeros past the resource,
-  // halo lanes' loads of the output read zeros and their stores are dropped
-  int xo[2], oo[2];
+  // halo lanes' loads of the output read zeros and their stores are dropped (unsigned: with a row's offset
+  // added, below 2^31 - 2^16, those lanes' offsets pass 2^31 but not 2^32)
+  unsigned xo[2], oo[2];
 #pragma unroll
   for (int i = 0; i < 2; i++) {
     const int xr = x0 - 1 + 16 * i + (lane >> 2), lx = 16 * i + l16, x = x0 - 1 + lx;
-    xo[i] = xr >= 0 && xr < Win ? (xr * cin + 4 * (lane & 3)) * 4 : 0x7ffffff0;
-    oo[i] = lx >= 1 && lx <= CR_COLS && x < Win && n < p.N ? ((UP ? 2 * x : x) * (int)p.ldc + n) * 4 : 0x7fff0000;
+    xo[i] = xr >= 0 && xr < Win ? (xr * cin + 4 * (lane & 3)) * 4 : 0x7ffffff0u;
+    oo[i] = lx >= 1 && lx <= CR_COLS && x < Win && n < p.N ? ((UP ? 2 * x : x) * (int)p.ldc + n) * 4 : 0x7fff0000u;
   }
   f32x4 raw[AHEAD][2][2];  // slot d: the next step d, d + AHEAD, ... of a row (nst % AHEAD == 0)
   auto load = [&](int y, int st, f32x4 (&v)[2][2]) __attribute__((always_inline)) {
@@ -567,7 +568,7 @@ __global__ __launch_bounds__(512, 2) void conv3x3_rows_kernel(TGemmArgs p, int R
   if (p.bias && n < p.N)
 #pragma unroll
     for (int r = 0; r < 4; r++) bias[r] = p.bias[n + r];
-  const int row_bytes = p.W * (int)p.ldc * 4;  // of the output
+  const unsigned row_bytes = p.W * (int)p.ldc * 4;  // of the output
 
   // UP: the row's products P, and the previous row's S[0] and S[0] + S[1] ([tile][even, odd]).
   // Plain: P[3 ty + tx] are the column accumulators of output row y + 1 - ty.
@@ -654,7 +655,7 @@ __global__ __launch_bounds__(512, 2) void conv3x3_rows_kernel(TGemmArgs p, int R
         }
       };
       const auto put = [&](int i, int e, int row, f32x4 v) __attribute__((always_inline)) {
-        const int vo = oo[i] + row * row_bytes + e * (int)p.ldc * 4;
+        const unsigned vo = oo[i] + row * row_bytes + e * (int)p.ldc * 4;
         v = v + bias;
         if (p.resid) v = cr_load(ro, vo, 0) + v;
         cr_store(ro, vo, v);
