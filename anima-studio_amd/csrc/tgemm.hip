@@ -689,18 +689,19 @@ __global__ __launch_bounds__(512, 2) void conv3x3_rows_kernel(TGemmArgs p, int R
 static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 // Rows per strip of conv3x3_rows_kernel: an XCD's workgroups run in rounds of one per CU, and each
-// takes R + 2 rows' products.  Returns the cost, rounds * (R + 2).
-static int64_t conv3x3_rows_strip(int num_cus, int64_t cols, int Hin, int ncg, int tpw, int* R) {
+// takes R + 2 rows' products; R with the smallest rounds * (R + 2).
+static int conv3x3_rows_strip(int num_cus, int64_t cols, int Hin, int ncg, int tpw) {
   const int64_t cus = num_cus >= 8 ? num_cus / 8 : 1;
   int64_t bc = -1;
+  int R = 1;
   for (int r = 1; r <= 256 && r <= Hin; r++) {
     const int64_t ntg = (cols * ((Hin + r - 1) / r) + tpw - 1) / tpw, wgs = (ntg + 7) / 8 * ncg, cost = (wgs + cus - 1) / cus * (r + 2);
     if (bc < 0 || cost <= bc) {
       bc = cost;
-      *R = r;
+      R = r;
     }
   }
-  return bc;
+  return R;
 }
 
 int conv3x3_launch(anima_ctx* c, const anima_conv_desc* d) {
@@ -741,13 +742,13 @@ int conv3x3_launch(anima_ctx* c, const anima_conv_desc* d) {
       in_bytes < (1LL << 31) - 65536 && out_bytes < (1LL << 31) - 65536) {
     const int bn = d->cin * 32 <= CR_MAXK && d->cout > 16 ? 32 : 16, tpw = 8 / (bn / 16);
     const int ncol = (Win + CR_COLS - 1) / CR_COLS, ncg = (d->cout + bn - 1) / bn;
-    int R = 1;
-    conv3x3_rows_strip(c->num_cus, (int64_t)d->B * ncol, Hin, ncg, tpw, &R);
+    const int R = conv3x3_rows_strip(c->num_cus, (int64_t)d->B * ncol, Hin, ncg, tpw);
     const int nstrip = (Hin + R - 1) / R;
     const int64_t ntask = (int64_t)d->B * ncol * nstrip, ntg = (ntask + tpw - 1) / tpw, blocks = (ntg + 7) / 8 * 8 * ncg;
     if (ntask <= 0x7ffffff && blocks <= 0x7fffffff) {
       const dim3 grid((unsigned)blocks);
-      Launch L(c, d->up ? "conv3x3.up" : "conv3x3", 2.0 * M * d->cout * 9.0 * d->cin, 0.0);
+      // (an upsampling conv takes its products at the input's resolution)
+      Launch L(c, d->up ? "conv3x3.up.rows" : "conv3x3.rows", 2.0 * d->B * Hin * Win * d->cout * 9.0 * d->cin, 0.0);
 #define CRA(U, S, BN, A) hipLaunchKernelGGL((conv3x3_rows_kernel<U, S, BN, A>), grid, dim3(512), 0, c->stream, p, R, ncol, nstrip, ncg, (int)ntask)
 #define CRB(U, S, BN)                     \
   {                                       \
@@ -777,7 +778,7 @@ int conv3x3_launch(anima_ctx* c, const anima_conv_desc* d) {
       (int64_t)d->B * (d->H / CT_TH) * (d->W / CT_TW) <= 0x7fffffff && (d->cout + bn - 1) / bn <= 65535) {
     // spatial tiles with the input halo in LDS
     const dim3 grid((unsigned)((int64_t)d->B * (d->H / CT_TH) * (d->W / CT_TW)), (unsigned)((d->cout + bn - 1) / bn));
-    Launch L(c, d->up ? "conv3x3.up" : "conv3x3", 2.0 * M * d->cout * 9.0 * d->cin, 0.0);
+    Launch L(c, d->up ? "conv3x3.up.tile" : "conv3x3.tile", 2.0 * M * d->cout * 9.0 * d->cin, 0.0);
 #define CTL(S, BN) hipLaunchKernelGGL((conv3x3_tile_kernel<S, CT_NW, BN>), grid, dim3(64 * CT_NW), 0, c->stream, p)
     if (bn == 96) {
       if (split) CTL(true, 96);

@@ -1,8 +1,8 @@
 // Qwen-Image (Wan 2.1) VAE decoder for single images on the gfx950 op layer, NHWC activations.
 // Restates app/models/vae.js (load 10-36, resblock 42-56, decode 59-113) on this build's ops:
-// conv3x3 as an implicit GEMM on the bf16 matrix cores (fused 2x nearest upsample and residual),
+// conv3x3 on the bf16 matrix cores (fused 2x nearest upsample and residual),
 // the channel norm kernel, the 1x1 convolutions as bf16-weight linears, and the single-head
-// 384-dim spatial attention on the chunked attention path.  The causal 3D convolutions arrive
+// 384-dim spatial attention (a fused kernel).  The causal 3D convolutions arrive
 // collapsed to 2D in OHWI layout (tools/build_assets.py:160-180).
 // Node-12 syntax only.
 

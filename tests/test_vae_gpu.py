@@ -61,8 +61,8 @@ CONV_CASES = [  # B, H, W (output), cin, cout, up, resid
     (2, 13, 11, 96, 3, False, True),
     (1, 32, 24, 192, 96, True, False),
     (1, 20, 20, 384, 192, True, True),
-    # spatial tiles (16 x 32 pixels x 96 channels, input halo in LDS): borders, several tiles and
-    # images, residual, upsample, several channel steps and column tiles
+    # by rows, and spatial tiles for the head (16 x 32 pixels, input halo in LDS): borders, several images,
+    # residual, upsample, several channel steps
     (2, 32, 64, 96, 96, False, True),
     (1, 32, 32, 192, 192, True, False),
     (1, 16, 32, 384, 384, False, False),
@@ -83,6 +83,42 @@ CONV_CASES = [  # B, H, W (output), cin, cout, up, resid
 @pytest.mark.parametrize("case", CONV_CASES)
 @pytest.mark.parametrize("precision", ["fp32", "bf16"])
 def test_conv3x3_matches_float64(case, precision):
+    run_conv(case, precision)
+
+
+CONV_KERNELS = [  # B, H, W (output), cin, cout, up, resid; the kernel
+    # by rows: one column, 30-column tiles short of and past a boundary, odd heights, channels that are no multiple of 16
+    ((1, 5, 1, 32, 20, False, True), "conv3x3.rows"),
+    ((3, 7, 29, 32, 36, False, False), "conv3x3.rows"),
+    ((1, 9, 31, 288, 96, False, True), "conv3x3.rows"),
+    ((1, 33, 61, 96, 20, False, True), "conv3x3.rows"),
+    ((2, 1, 30, 64, 16, False, False), "conv3x3.rows"),
+    ((2, 34, 122, 96, 48, True, True), "conv3x3.up.rows"),
+    # spatial tiles, with 96 and with 32 columns
+    ((1, 32, 32, 416, 96, False, True), "conv3x3.tile"),
+    ((1, 16, 64, 512, 192, True, False), "conv3x3.up.tile"),
+    ((2, 16, 32, 64, 3, False, True), "conv3x3.tile"),
+    ((1, 32, 32, 32, 30, True, False), "conv3x3.up.tile"),
+    # the implicit GEMM
+    ((1, 20, 24, 416, 96, False, True), "conv3x3"),
+    ((1, 12, 12, 48, 8, True, False), "conv3x3.up"),
+]
+
+
+@pytest.mark.parametrize("case,kernel", CONV_KERNELS)
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+def test_conv3x3_kernels(case, kernel, precision):
+    """Each 3x3 kernel where the dispatch takes it (the profiler's name), against float64; the profiler counts the
+    products of an upsampling conv by rows at the input's resolution."""
+    rep = run_conv(case, precision)
+    B, H, W, cin, cout, up, _ = case
+    assert list(rep) == [kernel], rep
+    flops = 2.0 * B * H * W * cout * 9 * cin / (4 if kernel == "conv3x3.up.rows" else 1)
+    assert abs(rep[kernel]["flops"] - flops) <= 1e-5 * flops
+
+
+def run_conv(case, precision):
+    """One 3x3 convolution against float64; returns the profiler's report by name."""
     from oracle import vae_ref
 
     m = amd()
@@ -98,7 +134,9 @@ def test_conv3x3_matches_float64(case, precision):
     with m.Context() as ctx:
         dx, dw, db = ctx.upload(x), ctx.upload(bf16_bits(w)), ctx.upload(bias)
         do = ctx.upload(c0) if resid else ctx.empty((B, H, W, cout))
+        ctx.profile(True)
         ctx.conv3x3(dx, dw, do, B=B, H=H, W=W, cin=cin, cout=cout, up=up, bias=db, resid=resid, precision=prec)
+        rep = {r["name"]: r for r in ctx.profile_report()}
         got = do.numpy()
         for b in (dx, dw, db, do):
             b.release()
@@ -107,6 +145,7 @@ def test_conv3x3_matches_float64(case, precision):
         ref = ref + c0
     r, _ = report(f"conv3x3 {case} {precision} vs float64", got, ref)
     assert r <= (3e-5 if precision == "fp32" else 1e-2)
+    return rep
 
 
 ATTN_CASES = [  # B, Lq, Lk, H, group, D, kv_len
