@@ -2,11 +2,11 @@
 
   * channel norm (app/gpu/kernels.js:62-89 mode 1) bit-exact against the C oracle, and within 1e-6
     with the SiLU (exp rounding);
-  * conv3x3 (implicit GEMM on the bf16 matrix cores, fused 2x upsample, bias, residual) against the
+  * conv3x3 (on the bf16 matrix cores, fused 2x upsample, bias, residual) against the
     float64 convolution (oracle/vae_ref.py, pinned by a direct loop): fp32 precision (activations as
     two bf16 terms) rel L2 <= 3e-5, bf16 <= 1e-2;
-  * attention with head dim 384 on the chunked path (app/gpu/ops.js:177-207) against float64,
-    including several score chunks, B = 2 with valid key lengths and GQA heads;
+  * attention with head dim 384 (fused) and others on the chunked path (app/gpu/ops.js:177-207) against
+    float64, including several score chunks, B = 2 with valid key lengths and GQA heads;
   * VAEDecoder.decode through the JS host against the float64 decoder on the same seeded weights:
     fp32 precision rel L2 <= 1e-3 with RGBA bytes within 1, bf16 precision reported and <= 5e-2.
 """
@@ -20,7 +20,7 @@ import numpy as np
 import pytest
 
 import oracle as orc
-from helpers import RUN_CASE, amd, report
+from helpers import RUN_CASE, amd, ran, report
 
 pytestmark = pytest.mark.gpu
 torch = pytest.importorskip("torch")
@@ -151,8 +151,12 @@ def run_conv(case, precision):
 ATTN_CASES = [  # B, Lq, Lk, H, group, D, kv_len
     (1, 300, 300, 1, 1, 384, None),
     (2, 256, 200, 2, 2, 384, [200, 77]),
-    (1, 2304, 16384, 1, 1, 384, None),  # one 2304 x 16384 score chunk
+    (1, 2304, 16384, 1, 1, 384, None),
     (1, 96, 150, 3, 1, 96, None),
+    # the chunked path with batches, grouped heads, ragged valid keys; rows of 16 / 32 / 64 scores per thread
+    (2, 130, 3000, 4, 2, 96, [3000, 1023]),
+    (2, 70, 6000, 2, 1, 96, [6000, 4097]),
+    (2, 129, 10000, 4, 4, 32, [10000, 8200]),
     # the fused 384-dim kernel: one query and key, one block and its edges, key splits with remainders and
     # batch elements shorter than a split
     (1, 1, 1, 1, 1, 384, None),
@@ -176,8 +180,9 @@ def test_chunked_attention_matches_float64(case, precision):
     print(f"[case] chunked attention {case} {precision}", flush=True)
     with m.Context() as ctx:
         dq, dk, dv, do = ctx.upload(q), ctx.upload(k), ctx.upload(v), ctx.empty((B, Lq, H * D))
-        ctx.attention(q=dq, k=dk, v=dv, o=do, B=B, Lq=Lq, Lk=Lk, H=H, D=D, ldq=H * D, ldk=Hk * D, ldv=Hk * D,
-                      group=group, kv_len=kv_len, precision=prec)
+        names = ran(ctx, lambda: ctx.attention(q=dq, k=dk, v=dv, o=do, B=B, Lq=Lq, Lk=Lk, H=H, D=D, ldq=H * D, ldk=Hk * D,
+                                               ldv=Hk * D, group=group, kv_len=kv_len, precision=prec))
+        assert ("attn.384" if D == 384 else "attn.chunk.softmax") in names, names
         got = do.numpy()
         for b in (dq, dk, dv, do):
             b.release()
@@ -236,11 +241,11 @@ def _attn_rows_f64(q, k, v, rows, D, causal, n=None):
     return np.array(out)
 
 
-@pytest.mark.parametrize("D", [64, 96])
+@pytest.mark.parametrize("D", [64, 96, 384])
 @pytest.mark.parametrize("precision", ["fp32", "bf16"])
 def test_chunked_attention_causal_gqa(D, precision):
     """The causal mask (app/gpu/ops.js:196, kernels.js:49: limit = min(cols, row + 1)) on the
-    chunked path (D = 96) and on the flash kernels with zero-padded operands (D = 64), with GQA (4
+    chunked path (D = 96, and 384, which only without the mask runs fused) and on the flash kernels with zero-padded operands (D = 64), with GQA (4
     query heads over 2 kv heads), B = 2 with a ragged valid key length, and Lq != Lk: every query
     row against a float64 restatement."""
     m = amd()
