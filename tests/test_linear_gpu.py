@@ -267,13 +267,13 @@ def w4_path(ctx):
 
 @pytest.mark.parametrize("kind,path", [("i8", "-"), ("w4", "scratch"), ("w4", "in_gemm")])
 def test_256_tile_kernel_ragged_edges(ctx, w4_path, kind, path):
-    """M=4500, N=4100: 18 x 17 tiles of 256 (the 256x256 persistent kernel), partial last row
-    and column tiles (rows / columns past the edge read as zero through the buffer bounds; W4
-    rows past N decode to zero), and a last group of 2 row tiles in the kernel's tile order
-    (groups of 4); gated residual + bias epilogue and the int32 accumulators bit-exact on
+    """M=4500, N=4100: 18 x 17 tiles of 256, partial last row and column tiles (rows / columns past the
+    edge read as zero through the buffer bounds; W4 rows past N decode to zero), and a last group of 2
+    row tiles in the 256x256 kernel's tile order (groups of 4).  W4 decoded in the GEMM runs that
+    kernel, the int8 weight and the scratch grid 128x128 tiles; gated residual + bias epilogue and the int32 accumulators bit-exact on
     sampled rows, including the last ones, and the accumulator checksums over the whole
     product.  W4 both ways: unpacked into the scratch grid and inside the GEMM."""
-    case(f"256x256-tile kernel M=4500 N=4100 K=1024 gated + bias {kind} {path}")
+    case(f"large tiles M=4500 N=4100 K=1024 gated + bias {kind} {path}")
     w4_path(path)
     m = amd()
     M, K, N = 4500, 1024, 4100
@@ -341,7 +341,7 @@ def test_256_tile_kernel_w4_every_srel(ctx, w4_path, K, path):
                                         (1537, 2048, 2112, "w4"), (2200, 2052, 2112, "i8"), (2240, 8192, 320, "w4"),
                                         (7904, 2048, 2112, "i8")])
 def test_int8_tile_sizes(ctx, M, N, K, kind):
-    """Every tile the int8 products choose from, with remainders in rows, columns and k: exact int32 sums, and the
+    """int8 products over the range of sizes, with remainders in rows, columns and k: exact int32 sums, and the
     fp32 residual epilogue bit for bit ((acc * s_x) * s_w added to C)."""
     m = amd()
     case(f"int8 tiles M={M} N={N} K={K} {kind}")
@@ -457,10 +457,10 @@ def test_int8_tile_choice(ctx, M, N, K, epi, lora, tile):
 
 @pytest.mark.parametrize("act,epi", [("gelu", 0), ("silu", 1)])
 def test_256_tile_kernel_activation_epilogues(ctx, act, epi):
-    """The 256x256 kernel with GELU (store) and SiLU (residual add) epilogues at M=4000, N=4100:
+    """Large tiles with GELU (store) and SiLU (residual add) epilogues at M=4000, N=4100:
     accumulators exact (checksums + sampled rows), activations within 1e-6 relative of the
     oracle's correctly rounded formula (the device uses its 1-ulp reciprocal and exp2)."""
-    case(f"256x256-tile kernel M=4000 N=4100 K=1024 {act} epi={epi}")
+    case(f"activations M=4000 N=4100 K=1024 {act} epi={epi}")
     m = amd()
     M, K, N = 4000, 1024, 4100
     x = orc.randn(97, M * K).reshape(M, K)
@@ -479,6 +479,87 @@ def test_256_tile_kernel_activation_epilogues(ctx, act, epi):
     ref = orc.linear_epilogue(ref_acc, sx[rows], sw, act=1 if act == "gelu" else 2, epi=epi, c=resid[rows])
     g = got[rows]
     assert rel_l2(g, ref) < 1e-6 and np.max(np.abs(g - ref)) <= 1e-6 * np.max(np.abs(ref)), report(act, g, ref)
+
+
+@pytest.mark.parametrize("M,N,K,kind,epi,act,extra,kernel", [
+    # 256x256, remainders of 60 rows / columns (and 164 / 220, 148 / 4 with several tiles per workgroup)
+    (3900, 3900, 1024, "i8", "gated", "none", "bias", "gemm.i8.256x256"),
+    (3900, 3900, 1024, "i8", "gated", "none", "bias add", "gemm.i8.256x256"),
+    (8100, 4060, 1024, "i8", "resid", "silu", "", "gemm.i8.256x256"),
+    (4500, 4100, 192, "i8", "store", "gelu", "bias", "gemm.i8.256x256"),
+    (4500, 4100, 64, "w4", "store", "none", "bias", "gemm.i8.256x256"),
+    (3900, 3900, 192, "w4", "resid", "none", "", "gemm.i8.256x256"),
+    (3900, 3900, 1024, "i8", "gated", "none", "bias lora48", "gemm.i8.256x256"),
+    (8100, 4060, 1024, "i8", "store", "gelu", "lora16", "gemm.i8.256x256"),
+    (3900, 3840, 1024, "w4", "resid", "none", "lora32/768", "gemm.i8.256x256"),
+    # the smaller tiles, K % 128 = 64
+    (1000, 2052, 1088, "i8", "gated", "none", "bias add", "gemm.i8.128x128"),
+    (2200, 2052, 2112, "i8", "gated", "silu", "bias", "gemm.i8.256x128"),
+    (777, 2044, 320, "w4", "gated", "none", "bias add", "gemm.i8.64x128"),
+    (200, 2044, 192, "i8", "store", "gelu", "bias add", "gemm.i8.32x64"),
+    (700, 2052, 1088, "i8", "store", "none", "bias lora48", "gemm.i8.64x128"),
+    (4500, 4100, 192, "i8", "gated", "none", "bias lora48", "gemm.i8.128x128"),
+    (2200, 2052, 2112, "w4", "resid", "none", "lora16", "gemm.i8.256x128"),
+    (777, 1536, 320, "i8", "gated", "gelu", "bias lora32/384", "gemm.i8.64x128"),
+    # the LoRA term added: rank blocks that split a tile, a gate that is not 16-byte aligned
+    (1000, 1152, 320, "i8", "gated", "none", "bias lora32/192", "gemm.i8.64x128"),
+    (200, 2048, 192, "i8", "gated", "none", "bias lora48", "gemm.i8.general")])
+def test_int8_kernels(ctx, M, N, K, kind, epi, act, extra, kernel):
+    """Each int8 kernel with each epilogue it has, the kernel asserted by its profiler name: exact int32 sums (checksums
+    over the product, sampled rows), the epilogue bit for bit, 1e-6 with an activation, rel L2 2e-6 with a LoRA term
+    (against the oracle epilogue fed the float64 term)."""
+    case(f"int8 kernels M={M} N={N} K={K} {kind} {epi} {act} {extra}")
+    m = amd()
+    rng = np.random.default_rng(M + N + K)
+    qx = rng.integers(-127, 128, size=(M, K), dtype=np.int8)
+    sx = rng.uniform(0.5, 1.5, M).astype(np.float32) / 127
+    bias = (0.1 * rng.standard_normal(N)).astype(np.float32) if "bias" in extra else None
+    b = ctx.upload(bias) if bias is not None else None
+    if kind == "i8":
+        qw, sw = int8_weight(7, N, K)
+        W = m.weight(m.W_I8, N, K, ctx.upload(qw), scale=ctx.upload(sw), bias=b)
+    else:
+        codes, srel, sw = w4_weight(7, N, K)
+        qw = orc.w4_decode(codes, srel, FIXED_LUT, N, K)
+        W = m.weight(m.W_W4, N, K, ctx.upload(codes), scale=ctx.upload(sw), srel=ctx.upload(srel), codebook=ctx.upload(FIXED_LUT), bias=b)
+    gate = rng.standard_normal(2 * N + 4).astype(np.float32)
+    g_off = N + 1 if "general" in kernel else (N + 3) // 4 * 4
+    c0 = rng.standard_normal((M, N)).astype(np.float32)
+    rows = np.unique(np.concatenate([np.arange(0, 4), rng.choice(M, 12, replace=False), np.arange(M - 8, M)]))
+    kw, add, lora = {}, None, [x for x in extra.split() if x.startswith("lora")]
+    if "add" in extra:
+        add = rng.standard_normal((M, N + 4)).astype(np.float32)
+        kw = dict(add=ctx.upload(add), ld_add=N + 4)
+        add = np.ascontiguousarray(add[rows, :N])
+    elif lora:
+        R, cols = (int(x) for x in (lora[0][4:] + "/0").split("/")[:2])
+        nb = N // cols if cols else 1
+        xa = (0.5 * rng.standard_normal((M, nb * R + 4))).astype(np.float32)
+        Bm = (0.05 * rng.standard_normal((N, R))).astype(np.float32)
+        planes = ctx.empty(3 * N * R, np.uint16)
+        ctx.split3_bf16(ctx.upload(Bm), planes, N * R)
+        kw = dict(lora_xa=ctx.upload(xa), ld_lora_xa=nb * R + 4, lora_b=planes, lora_r=R, lora_cols=cols)
+        blk = np.arange(N) // (cols or N)
+        add = np.einsum("mnr,nr->mn", xa[rows].astype(np.float64)[:, blk[:, None] * R + np.arange(R)], Bm.astype(np.float64)).astype(np.float32)
+    out, acc = ctx.upload(c0), ctx.empty((M, N), np.int32)
+    e = {"store": m.EPI_STORE, "resid": m.EPI_RESID, "gated": m.EPI_GATED}[epi]
+    names = ran(ctx, lambda: ctx.linear(W, M, out, xq=ctx.upload(qx), xs=ctx.upload(sx), epilogue=e, act=act, gate=ctx.upload(gate),
+                                        gate_off=g_off, acc_out=acc, **kw))
+    assert kernel in names, names
+    assert ("gemm.f32s3" in names) == bool(lora and ("/192" in extra or "general" in kernel)), names
+    got = acc.numpy()
+    assert checksums_ok(qx, qw, got)
+    ref_acc = orc.gemm_i8(qx[rows], qw)
+    assert np.array_equal(got[rows], ref_acc)
+    ref = orc.linear_epilogue(ref_acc, sx[rows], sw, bias=bias, act={"none": 0, "gelu": 1, "silu": 2}[act], epi=e, gate=gate,
+                              g_off=g_off, c=c0[rows] if epi != "store" else None, add=add)
+    g = out.numpy()[rows]
+    if lora:
+        assert report("LoRA", g, ref)[0] <= 2e-6
+    elif act != "none":
+        assert rel_l2(g, ref) < 1e-6 and np.max(np.abs(g - ref)) <= 1e-6 * np.max(np.abs(ref)), report(act, g, ref)
+    else:
+        assert np.array_equal(g, ref), report(epi, g, ref)
 
 
 @pytest.mark.parametrize("act", ["gelu", "silu"])
@@ -562,7 +643,7 @@ def test_bf16_weight_split_kernel(ctx, M, K, N, epi):
 @pytest.mark.parametrize("M", [4000, 200])
 def test_linear_add_term(ctx, M):
     """The optional fp32 add term (the LoRA delta input of gemm.js:189) after the bias: M=4000
-    runs the 256-tile kernel (16-byte add rows, ld_add > N), M=200 the 128-tile kernel; gated
+    runs 128x128 tiles (16-byte add rows, ld_add > N), M=200 32x64 tiles; gated
     epilogue, bit-exact against the oracle epilogue."""
     case(f"linear add term M={M} N=4100 K=1024 gated + bias")
     m = amd()
@@ -597,8 +678,7 @@ def test_linear_lora_epilogue(ctx, M, epi, act):
     lora_xa / lora_b / lora_r): y += xa[m] . B[n] after the bias, before the activation / gate
     (ops.js:55-87 with the scale folded into B).  xa [M, R] fp32 with ld > R, B [N, R] as three
     bf16 planes (anima_split3_bf16), R = 48 (three 16-k slices); N = 4100 leaves a partial column
-    tile.  M = 4000 runs the 256-tile kernel with the product inside its epilogue, M = 200 the
-    128-tile kernel with the product as an add term.  Against the oracle epilogue fed the float64
+    tile.  The product runs inside the epilogue of 128x128 (M = 4000) and 64x128 tiles.  Against the oracle epilogue fed the float64
     delta (rounded to fp32): rel-L2 <= 2e-6; the int32 accumulators bit-exact."""
     case(f"linear LoRA epilogue M={M} {epi} act={act}")
     m = amd()
@@ -636,10 +716,8 @@ def test_linear_lora_epilogue(ctx, M, epi, act):
 def test_linear_lora_block_diagonal(ctx, M, N, cols):
     """Block-diagonal LoRA ranks (lora_cols: a stacked projection whose column blocks carry their
     own ranks, e.g. q / k / v): column n adds xa[m, (n // cols) * R + k] * B[n, k], B holding only
-    each block's R = 32 ranks.  cols = 1024 runs the product inside the 256-tile kernel's
-    epilogue (a tile lies in one block); cols = 384 splits tiles and M = 200 runs the 128-tile
-    kernel, both taking the product as an add term, one split-bf16 product per block over its
-    rows of the B planes.  Against the oracle epilogue fed the float64 delta: rel-L2 <= 2e-6."""
+    each block's R = 32 ranks, inside the epilogue (every tile of 128 columns lies in one block).
+    Against the oracle epilogue fed the float64 delta: rel-L2 <= 2e-6."""
     case(f"linear LoRA block-diagonal M={M} N={N} cols={cols}")
     m = amd()
     K, R = 1024, 32

@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 import oracle as orc
-from helpers import amd, report
+from helpers import amd, ran, report
 from test_linear_gpu import FIXED_LUT, int8_weight, w4_weight
 
 pytestmark = pytest.mark.gpu
@@ -130,8 +130,7 @@ def run_linear_qkv_case(ctx, m, kind, B, Hp, Wp, H, K, bias):
 def test_linear_qkv_lora(ctx, kind, cols):
     """The fused QKV epilogue with the LoRA term (anima_linear_desc lora_*): Q and the K / V operands
     bit-identical to the LoRA linear's fp32 output converted by anima_attention_prepare_kv.
-    B = 2, 48 x 48 tokens (M = 4608: the plain linear also runs the product inside its epilogue,
-    as it does from one 256 x 256 tile per CU up), H = 16, K = 2048; rank 32 per q / k / v block
+    B = 2, 48 x 48 tokens (M = 4608; the plain linear also runs the product inside its epilogue), H = 16, K = 2048; rank 32 per q / k / v block
     (lora_cols = 2048), or one rank-48 block over all columns (lora_cols = 0)."""
     case(f"linear_qkv LoRA {kind} cols={cols}")
     m = amd()
@@ -224,6 +223,78 @@ def test_linear_qkv_prepared_q(ctx, kind, Hp, Wp):
     err = np.abs(got - want) / np.maximum(np.abs(want), 1e-3)
     assert err.max() <= 2.0 ** -8 + 1e-5, err.max()
     for x in wbufs + [xq, xs, dqn, dkn, dcs, ref, prep_ref, qp, prep, o1, o2]:
+        x.release()
+
+
+@pytest.mark.parametrize("B,Hp,Wp,H,K,cols,tile", [
+    (1, 16, 16, 16, 2112, 0, "64x128"), (2, 16, 32, 16, 2112, 0, "256x128"), (2, 32, 32, 16, 2048, 0, "128x128"), (2, 33, 64, 16, 2048, 0, "256x256"),
+    (1, 16, 16, 16, 2112, 2048, "64x128"), (2, 16, 32, 16, 2112, 6144, "256x128"), (2, 32, 32, 16, 2048, 2048, "128x128"),
+    (1, 8, 8, 2, 65600, 256, "256x256")])
+@pytest.mark.parametrize("prepared", [False, True])
+def test_linear_qkv_tiles(ctx, B, Hp, Wp, H, K, cols, tile, prepared):
+    """The operand epilogue on every tile (asserted by the profiler name), with fp32 and prepared Q and with a LoRA term
+    (cols: its rank blocks): K / V bytes and Q bits of the plain linear and prepare_kv, and with prepared Q the attention's
+    output bit for bit."""
+    case(f"linear_qkv tile {tile} B={B} {Hp}x{Wp} H={H} K={K} lora={cols} prepared={prepared}")
+    m = amd()
+    L = Hp * Wp
+    M, N = B * L, 3 * H * HD
+    W, wbufs = make_weight(ctx, m, "i8", 990 + K, N, K, True)
+    rng = np.random.default_rng(L + K)
+    xq = ctx.upload(rng.integers(-127, 128, size=(M, K), dtype=np.int8))
+    xs = ctx.upload(rng.uniform(0.002, 0.02, M).astype(np.float32))
+    lk = {}
+    if cols:
+        R, nb = 32, N // cols
+        planes = ctx.empty(3 * N * R, np.uint16)
+        ctx.split3_bf16(ctx.upload((0.05 * rng.standard_normal((N, R))).astype(np.float32)), planes, N * R)
+        lk = dict(lora_xa=ctx.upload((0.5 * rng.standard_normal((M, nb * R))).astype(np.float32)), ld_lora_xa=nb * R, lora_b=planes,
+                  lora_r=R, lora_cols=cols)
+    qn, kn = (ctx.upload((1 + 0.02 * orc.randn(s_, HD)).astype(np.float32)) for s_ in (991, 992))
+    cs = ctx.upload(orc.dit_rope_table(Hp, Wp))
+    nbytes = m.Context.attention_kv_bytes(B, H, L, m.PREC_BF16)
+    ref, prep_ref, prep = ctx.empty((M, N)), ctx.empty(nbytes, np.uint8), ctx.empty(nbytes, np.uint8)
+    ctx.linear(W, M, ref, xq=xq, xs=xs, **lk)
+    common = dict(B=B, Lq=L, Lk=L, H=H, D=HD, ldq=N, ldk=N, ldv=N, precision=m.PREC_BF16, rope_cs=cs, rope_sin_off=L * 64)
+    ctx.attention(q=ref, k=ref, v=ref, o=ref, prepare_into=prep_ref, k_norm=kn, k_off=H * HD, v_off=2 * H * HD, **common)
+    q, qp = ctx.empty((M, H * HD)), ctx.empty(M * H * HD, np.uint16)
+    names = ran(ctx, lambda: ctx.linear_qkv(W, M, None if prepared else q, B=B, L=L, H=H, k_norm=kn, rope_cs=cs, rope_sin_off=L * 64,
+                                            kv_prep=prep, xq=xq, xs=xs, ldc=0 if prepared else H * HD,
+                                            **(dict(q_norm=qn, q_prep=qp) if prepared else {}), **lk))
+    assert names == {"gemm.i8_qkv." + tile}, names
+    assert np.array_equal(prep.numpy(), prep_ref.numpy())
+    if prepared:
+        o1, o2 = ctx.empty((M, H * HD)), ctx.empty((M, H * HD))
+        ctx.attention(q=ref, k=None, v=None, o=o1, kv_prep=prep_ref, q_norm=qn, **common)
+        ctx.attention(q=None, k=None, v=None, o=o2, kv_prep=prep, q_prep=qp, **common)
+        assert np.array_equal(o1.numpy(), o2.numpy())
+    else:
+        assert np.array_equal(q.numpy(), ref.numpy()[:, :H * HD])
+    for x in wbufs + [xq, xs, qn, kn, cs, ref, prep_ref, prep, q, qp]:
+        x.release()
+
+
+@pytest.mark.parametrize("M,K,tile", [(512, 1088, "64x128"), (1088, 2112, "128x128"), (2240, 2112, "256x128"), (4992, 2112, "256x256")])
+def test_linear_q_only_tiles(ctx, M, K, tile):
+    """A Q-only projection of 20 heads on every tile: the prepared values are within bf16 rounding of float64."""
+    case(f"linear_qkv Q-only tile {tile} M={M} K={K}")
+    m = amd()
+    H = 20
+    N = H * HD
+    W, wbufs = make_weight(ctx, m, "i8", 995, N, K, True)
+    rng = np.random.default_rng(M)
+    xq = ctx.upload(rng.integers(-127, 128, size=(M, K), dtype=np.int8))
+    xs = ctx.upload(rng.uniform(0.002, 0.02, M).astype(np.float32))
+    qn = (1 + 0.02 * orc.randn(996, HD)).astype(np.float32)
+    dqn, ref, qp = ctx.upload(qn), ctx.empty((M, N)), ctx.empty(M * N, np.uint16)
+    ctx.linear(W, M, ref, xq=xq, xs=xs)
+    names = ran(ctx, lambda: ctx.linear_qkv(W, M, None, B=1, L=M, H=H, xq=xq, xs=xs, q_norm=dqn, q_prep=qp))
+    assert names == {"gemm.i8_qkv." + tile}, names
+    q = ref.numpy().astype(np.float64).reshape(M, H, HD)
+    want = q / np.sqrt((q * q).mean(-1, keepdims=True) + 1e-6) * qn * (np.log2(np.e) / np.sqrt(HD))
+    err = np.abs(bf16_to_f32(qp.numpy().reshape(M, H, HD)) - want) / np.maximum(np.abs(want), 1e-3)
+    assert err.max() <= 2.0 ** -8 + 1e-5, err.max()
+    for x in wbufs + [xq, xs, dqn, ref, qp]:
         x.release()
 
 
