@@ -3,9 +3,9 @@
 //
 //   gemm_i8   C = epi((qx @ qw^T) * s_x[m] * s_w[n]) with v_mfma_i32_32x32x32_i8 (exact int32
 //             accumulation): gemm_i8_256 and the smaller tiles of gemm_i8_tile, chosen by size, on
-//             int8 weights (W4: on the unpacked grid); gemm_i8_kernel for unaligned rows, and for W4
-//             weights decoded inside a product that is not given the 256x256 tile: block tile
-//             128x128, k-tile 64, 4 waves of 64x64, double-buffered LDS with 80-byte rows
+//             int8 weights (W4: on the unpacked grid); gemm_i8_kernel for unaligned rows, rows of
+//             2^23 weights and more, and W4 weights decoded inside a product without a 256x256
+//             tile for every CU: block tile 128x128, k-tile 64, 4 waves of 64x64, double-buffered LDS with 80-byte rows
 //             (conflict-free 16-byte fragment reads).
 //             W4: the weight tile is decoded in the loader, nibble -> int8 grid value through a
 //             16-entry table per 16-weight group.  The table of a group depends only on its fp8

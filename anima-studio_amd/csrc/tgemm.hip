@@ -1062,8 +1062,8 @@ __global__ __launch_bounds__(256) void pv_sum_kernel(const float* part, int ks, 
 // needs one lane exchange, and its weights are the next product's operand as they stand (V^T's keys
 // are stored in that order: 0-3, 8-11, 4-7, 12-15 of each 16).  Queries too few for the CUs split the
 // keys, partial outputs (unnormalized, with the row's maximum and sum) combined afterwards.
-// Against the chunked path: 128 x 128 latents fp32 2656 -> 1067 us (1170 TFLOP/s of the three products; a
-// large library product reaches 1250), bf16 2000 -> 490; 64 x 64 193 -> 117 / 159 -> 76; 32 x 32 115 -> 60
+// Against the chunked path: 128 x 128 latents fp32 2645 -> 1075 us (this kernel 1055, 1173 TFLOP/s of the three
+// products; a large library product reaches 1250), bf16 2000 -> 490; 64 x 64 193 -> 117 / 159 -> 76; 32 x 32 115 -> 60
 // / 87 -> 44.
 constexpr int FA_D = 384, FA_KB = 32, FA_Q = 128, FA_NS = FA_D / 16, FA_NT = FA_D / 32, FA_MAXB = 64;
 
