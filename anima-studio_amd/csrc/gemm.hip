@@ -2248,7 +2248,7 @@ __global__ __launch_bounds__(128 * KG) void gemm_bf16_s3_kernel(F32WArgs a) {
 // us, 3072 x 1024 23.1 -> 17.2; at 43 tokens 8 to 10 us, most of it a launch and first loads).  LDS rows of 40 bf16 (80 bytes)
 // give conflict-free 16-byte fragment reads.  Epilogue and C^T layout of gemm_bf16_s3_kernel.
 constexpr int B3L_ROW = 40;
-template <int KG, int AHEAD>
+template <int KG, int AHEAD, bool SHORT = false>
 __global__ __launch_bounds__(256 * KG) void gemm_bf16_s3_lds_kernel(F32WArgs a) {
   constexpr int XS = 3 * 64 * B3L_ROW, WS = 128 * B3L_ROW, BUF = XS + WS;  // a step's x planes and weights
   __shared__ __attribute__((aligned(16))) bf16 smem[KG * 2 * BUF];
@@ -2277,6 +2277,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_bf16_s3_lds_kernel(F32WArgs a) 
     uint4 w[2];
   } sl[AHEAD];  // slot d: the next step d, d + AHEAD, ... (nch % AHEAD == 0)
   auto load = [&](int kc, Step& v) __attribute__((always_inline)) {  // (past the last step: that one again, unused)
+    if (SHORT && kc >= nch) return;  // (short rows: the loads past the end would be much of all)
     const int k0 = 32 * min(kc, nch - 1);
 #pragma unroll
     for (int i = 0; i < 2; i++) {
@@ -2669,15 +2670,15 @@ static void s3_lds_launch(anima_ctx* c, const F32WArgs& f, int ks) {
   const dim3 grid((f.N + 127) / 128, (f.M + 63) / 64, ks);
   const bool two = (int64_t)grid.x * grid.y * ks <= c->num_cus && f.K % 64 == 0;
   const int nch = f.K / 32 / (two ? 2 : 1);
-#define S3L(KG, A) hipLaunchKernelGGL((gemm_bf16_s3_lds_kernel<KG, A>), grid, dim3(256 * KG), 0, c->stream, f)
+#define S3L(...) hipLaunchKernelGGL((gemm_bf16_s3_lds_kernel<__VA_ARGS__>), grid, dim3(two ? 512 : 256), 0, c->stream, f)
   if (two) {
     if (nch % 4 == 0) S3L(2, 4);
     else if (nch % 2 == 0) S3L(2, 2);
     else S3L(2, 1);
-  } else {
-    if (nch % 4 == 0) S3L(1, 4);
-    else if (nch % 2 == 0) S3L(1, 2);
-    else S3L(1, 1);
+  } else {  // several workgroups per CU: four steps ahead took 5 to 15% longer than two
+    if (nch % 2) S3L(1, 1, true);
+    else if (nch <= 12) S3L(1, 2, true);  // (5420 x 808 x 128 16.5 -> 15.8 us; 1024 x 2304 x 2048 47.6 and 46.7 without)
+    else S3L(1, 2);
   }
 #undef S3L
 }
