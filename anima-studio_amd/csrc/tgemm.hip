@@ -280,8 +280,8 @@ static int tgemm_launch(anima_ctx* c, const TGemmArgs& p, int amode, int bmode, 
   return L.end();
 }
 
-// ---- conv3x3 on spatial tiles (the 3-channel head, and rows of more than 384 channels: what
-// conv3x3_rows_kernel below does not take): a workgroup (8 waves) computes a 16 x 32 block of output pixels
+// ---- conv3x3 on spatial tiles (the 3-channel head, more than 384 channels, and sizes of more than 192 where it is
+// shorter than conv3x3_rows_kernel below): a workgroup (8 waves) computes a 16 x 32 block of output pixels
 // for BN = 96 output channels (or one 32-wide column tile when cout <= 32: the 3-channel head).  Per step of 32 input channels the input halo it needs (18 x 34 pixels in
 // output coordinates, sampled through the 2x nearest upsample when up; zero outside the image) and
 // the 9 x 96 x 32 weights are copied once into LDS, so every input value is read from memory once
@@ -689,19 +689,42 @@ __global__ __launch_bounds__(512, 2) void conv3x3_rows_kernel(TGemmArgs p, int R
 static bool al16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
 // Rows per strip of conv3x3_rows_kernel: an XCD's workgroups run in rounds of one per CU, and each
-// takes R + 2 rows' products; R with the smallest rounds * (R + 2).
-static int conv3x3_rows_strip(int num_cus, int64_t cols, int Hin, int ncg, int tpw) {
+// takes R + 2 rows' products; R with the smallest cost, rounds * (R + 2).
+struct ConvStrip {
+  int R;
+  int64_t cost;
+};
+static ConvStrip conv3x3_rows_strip(int num_cus, int64_t cols, int Hin, int ncg, int tpw) {
   const int64_t cus = num_cus >= 8 ? num_cus / 8 : 1;
-  int64_t bc = -1;
-  int R = 1;
+  ConvStrip best{1, -1};
   for (int r = 1; r <= 256 && r <= Hin; r++) {
     const int64_t ntg = (cols * ((Hin + r - 1) / r) + tpw - 1) / tpw, wgs = (ntg + 7) / 8 * ncg, cost = (wgs + cus - 1) / cus * (r + 2);
-    if (bc < 0 || cost <= bc) {
-      bc = cost;
-      R = r;
-    }
+    if (best.cost < 0 || cost <= best.cost) best = {r, cost};
   }
-  return R;
+  return best;
+}
+
+// Whether the conv by rows (bn output channels per workgroup) is the shorter kernel.  It nearly always is; by measured
+// time per 32 input channels (us, fp32 / bf16 precision) it is not
+//   * on spatial tiles' sizes with more than 192 input channels, where half of its waves hold the same pixels: rows
+//     0.97 / 0.49 per unit of cost; tiles 11 + 4 / 7.6 + 2.8 times the share of the CUs in use, per round
+//     (384 channels fp32 256 x 256 426 us and 376, 256 x 128 253 and 180, 128 x 128 130 and 152);
+//   * on images of up to 8 columns, where most of a wave's 32 are empty: the implicit GEMM's 128 x 128 tiles
+//     (4096 x 1 pixels, 384 channels fp32 512 us and 124).
+static bool conv3x3_rows_shorter(int num_cus, const anima_conv_desc* d, bool split, int bn, int64_t cost) {
+  const float k = (float)(d->cin / 32), cus = (float)num_cus;
+  if (d->cout % 96 == 0 && d->H % CT_TH == 0 && d->W % CT_TW == 0) {
+    if (d->up || bn != 16) return true;
+    const int64_t n = (int64_t)d->B * (d->H / CT_TH) * (d->W / CT_TW) * (d->cout / 96), q = n / num_cus, rest = n % num_cus;
+    const float a = split ? 11.0f : 7.6f, b = split ? 4.0f : 2.8f;
+    return (split ? 0.97f : 0.49f) * (float)cost <= (float)q * (a + b) + (rest ? a + b * (float)rest / cus : 0.0f);
+  }
+  if ((d->up ? d->W / 2 : d->W) > 8) return true;
+  const int64_t n = (((int64_t)d->B * d->H * d->W + TG_BM - 1) / TG_BM) * ((d->cout + TG_BN - 1) / TG_BN), slots = (int64_t)num_cus * (split ? 2 : 4);
+  const int64_t q = n / slots, rest = n % slots;
+  const float gemm = (split ? 16.0f : 18.0f) * (float)q + (rest ? (split ? 8.8f : 7.0f) + (split ? 2.0f : 2.5f) * (float)rest / cus : 0.0f);
+  const float row = bn == 32 ? (d->up ? (split ? 1.2f : 0.85f) : (split ? 0.97f : 0.63f)) : (d->up ? (split ? 0.87f : 0.61f) : (split ? 0.85f : 0.53f));
+  return 0.85f * (3.0f + row * (float)cost * k) <= 10.0f + gemm * k;
 }
 
 int conv3x3_launch(anima_ctx* c, const anima_conv_desc* d) {
@@ -742,10 +765,10 @@ int conv3x3_launch(anima_ctx* c, const anima_conv_desc* d) {
       in_bytes < (1LL << 31) - 65536 && out_bytes < (1LL << 31) - 65536) {
     const int bn = d->cin * 32 <= CR_MAXK && d->cout > 16 ? 32 : 16, tpw = 8 / (bn / 16);
     const int ncol = (Win + CR_COLS - 1) / CR_COLS, ncg = (d->cout + bn - 1) / bn;
-    const int R = conv3x3_rows_strip(c->num_cus, (int64_t)d->B * ncol, Hin, ncg, tpw);
+    const auto [R, cost] = conv3x3_rows_strip(c->num_cus, (int64_t)d->B * ncol, Hin, ncg, tpw);
     const int nstrip = (Hin + R - 1) / R;
     const int64_t ntask = (int64_t)d->B * ncol * nstrip, ntg = (ntask + tpw - 1) / tpw, blocks = (ntg + 7) / 8 * 8 * ncg;
-    if (ntask <= 0x7ffffff && blocks <= 0x7fffffff) {
+    if (ntask <= 0x7ffffff && blocks <= 0x7fffffff && conv3x3_rows_shorter(c->num_cus, d, split, bn, cost)) {
       const dim3 grid((unsigned)blocks);
       // (an upsampling conv takes its products at the input's resolution)
       Launch L(c, d->up ? "conv3x3.up.rows" : "conv3x3.rows", 2.0 * d->B * Hin * Win * d->cout * 9.0 * d->cin, 0.0);

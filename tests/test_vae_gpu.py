@@ -99,7 +99,11 @@ CONV_KERNELS = [  # B, H, W (output), cin, cout, up, resid; the kernel
     ((1, 16, 64, 512, 192, True, False), "conv3x3.up.tile"),
     ((2, 16, 32, 64, 3, False, True), "conv3x3.tile"),
     ((1, 32, 32, 32, 30, True, False), "conv3x3.up.tile"),
+    ((1, 128, 256, 384, 96, False, True), "conv3x3.rows"),
+    ((1, 256, 128, 384, 384, False, False), "conv3x3.tile"),
     # the implicit GEMM
+    ((1, 4000, 1, 96, 384, False, True), "conv3x3"),
+    ((1, 4096, 4, 96, 384, True, False), "conv3x3.up"),
     ((1, 20, 24, 416, 96, False, True), "conv3x3"),
     ((1, 12, 12, 48, 8, True, False), "conv3x3.up"),
 ]
