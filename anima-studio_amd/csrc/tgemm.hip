@@ -1184,7 +1184,8 @@ __global__ __launch_bounds__(512, 2) void attn384_kernel(FaArgs a, int nitem) {
   f32x16 O[HT];
 #pragma unroll
   for (int i = 0; i < HT; i++) O[i] = f32x16{};
-  float m = -INFINITY, l = 0.0f;
+  // mf: m, or 0 while no score was finite: weights of zero then (as they are beside the finite scores of other blocks)
+  float m = -INFINITY, mf = 0.0f, l = 0.0f;
 
   if (nb > 0) {
     const char* src = a.kv + ((int64_t)b * (a.H / a.group) + h / a.group) * a.kv_head + (int64_t)kb0 * (2 * TB);
@@ -1257,6 +1258,7 @@ __global__ __launch_bounds__(512, 2) void attn384_kernel(FaArgs a, int nitem) {
       if (__any(mx > m)) {  // (rare once the first blocks are done)
         const float mn = fmaxf(m, mx), al = mx > m ? __builtin_amdgcn_exp2f(m - mn) : 1.0f;  // (m may be -inf still)
         m = mn;
+        mf = mn == -INFINITY ? 0.0f : mn;
         l = l * al;
 #pragma unroll
         for (int i = 0; i < HT; i++) O[i] = O[i] * al;
@@ -1264,8 +1266,6 @@ __global__ __launch_bounds__(512, 2) void attn384_kernel(FaArgs a, int nitem) {
       // the next block's scores beside this block's weights (after the last block: of the last again, unused)
       S = f32x16{};
       scores(S);
-      // no finite score so far: weights of zero (as they are beside the finite scores of other key blocks)
-      const float mf = m == -INFINITY ? 0.0f : m;
       bf16x8 ph[2], pl[2];
 #pragma unroll
       for (int s2 = 0; s2 < 2; s2++) {
