@@ -1155,7 +1155,7 @@ __global__ __launch_bounds__(256, 3 - KG) void attn_flash_fp32(FlashArgs a) {
   // causal: as in attn_flash_bf16 (lim: this lane's key limit; mlim: the workgroup's smallest)
   const int lim = a.causal ? min(Lk, qi + 1) : Lk;
   const int mlim = a.causal ? min(Lk, qt * BQ32<KG> + 1) : Lk;
-  const int nkb = a.causal ? min((Lk + BK - 1) / BK, (qt + 1) * (BQ32<KG> / BK)) : (Lk + BK - 1) / BK;
+  const int nkb = a.causal ? min((Lk + BK - 1) / BK, (min((qt + 1) * BQ32<KG>, a.Lq) + BK - 1) / BK) : (Lk + BK - 1) / BK;
 
   // k-step 4 g + e of the scores: dim 8 g + e in lane half 0, 8 g + 4 + e in half 1, so that a lane reads
   // its K values four steps at a time; lane keeps Q[qi][8 g + 4 hf + e] as qv[4 g + e]

@@ -363,6 +363,7 @@ def test_head_dim_64_flash_path(ctx, precision):
 
 @pytest.mark.parametrize("B,Lq,Lk,H,group,causal,kv_len,form", [
     (1, 4096, 64, 16, 1, 0, None, "attn.flash_fp32"), (1, 64, 60, 2, 1, 1, None, "attn.flash_fp32"),
+    (2, 6, 400, 4, 2, 1, [400, 3], "attn.flash_fp32"), (1, 64, 300, 2, 1, 1, None, "attn.flash_fp32"),
     (4, 300, 200, 16, 2, 0, [200, 64, 1, 130], "attn.flash_fp32"), (2, 1300, 512, 8, 1, 0, [449, 512], "attn.flash_fp32"),
     (1, 129, 200, 2, 1, 0, None, "attn.flash_fp32_2g"), (2, 65, 320, 4, 2, 0, [320, 63], "attn.flash_fp32_2g"),
     (1, 192, 192, 2, 1, 1, None, "attn.flash_fp32_2g"), (3, 130, 77, 2, 1, 1, [77, 70, 5], "attn.flash_fp32_2g")])
