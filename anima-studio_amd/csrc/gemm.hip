@@ -4,8 +4,8 @@
 //   gemm_i8   C = epi((qx @ qw^T) * s_x[m] * s_w[n]) with v_mfma_i32_32x32x32_i8 (exact int32
 //             accumulation): gemm_i8_256 and the smaller tiles of gemm_i8_tile, chosen by size, on
 //             int8 weights (W4: on the unpacked grid); gemm_i8_kernel for unaligned rows, rows of
-//             2^23 weights and more, and W4 weights decoded inside a product without a 256x256
-//             tile for every CU: block tile 128x128, k-tile 64, 4 waves of 64x64, double-buffered LDS with 80-byte rows
+//             2^23 weights and more, and W4 weights decoded inside a product of up to 32 rows:
+//             block tile 128x128, k-tile 64, 4 waves of 64x64, double-buffered LDS with 80-byte rows
 //             (conflict-free 16-byte fragment reads).
 //             W4: the weight tile is decoded in the loader, nibble -> int8 grid value through a
 //             16-entry table per 16-weight group.  The table of a group depends only on its fp8
@@ -2943,14 +2943,15 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
   // what is left).
   const bool vec = K < (1 << 23) && N % 4 == 0 && g.ldc % 4 == 0 && al(g.out, 16) && al(g.sw, 16) && (!g.bias || al(g.bias, 16)) &&
                    (g.epi != ANIMA_EPI_GATED || al(g.gate + g.gate_off, 16)) && (!g.add || (al(g.add, 16) && g.ld_add % 4 == 0));
-  // a 256x256 tile for every CU: of the two kernels that decode W4 codes, the 256x256 one takes these products (its
-  // decode runs beside the matrix cores: 4096 x 6144 x 2048 103 us, gemm_i8_kernel 163) and the other the rest
   const int64_t tiles256 = (int64_t)((N + 255) / 256) * ((M + 255) / 256);
-  const bool big = vec && tiles256 >= c->num_cus && tiles256 <= 0x7fffffff;
+  // of the two kernels that decode W4 codes, the 256x256 one runs its decode beside the matrix cores: shorter for all but
+  // few rows (2112 x 6144 x 4864 101 us, gemm_i8_kernel 230; 43 x 2048 x 64 10.2 and 18.8; 1 x 2048 x 2048 30.5 and 23.1)
+  const bool few = M <= (K > 4096 ? 64 : 32) || tiles256 > 0x7fffffff;
   void* grid8 = nullptr;
   bool w4k = w4;  // the GEMM unpacks W4 codes itself
-  // (the LoRA epilogue of a tile runs on the int8 grid: the in-GEMM unpack leaves it no registers)
-  if (w4 && vec && (lora ? big || c->w4_path == ANIMA_W4_GRID_SCRATCH
+  // (the LoRA epilogue of a tile runs on the int8 grid: the in-GEMM unpack leaves it no registers, and an add term
+  // takes more scratch and time than the grid)
+  if (w4 && vec && (lora ? !few || c->w4_path == ANIMA_W4_GRID_SCRATCH
                          : c->w4_path == ANIMA_W4_GRID_SCRATCH && !w4_few_rows(c, M, N, K))) {
     rc = w4_grid_scratch(c, W, g, &grid8);
     if (rc && rc != ANIMA_E_OOM) {
@@ -2961,7 +2962,9 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
     else (void)hipGetLastError();  // no memory for the grid: the codes are unpacked inside the GEMM
     rc = ANIMA_OK;
   }
-  const int tile = !vec ? -1 : !w4k ? gemm_i8_choose(c, M, N, K, lora ? GT_LORA : g.epi == ANIMA_EPI_STORE ? GT_STORE : GT_RESID) : big && !lora ? (int)GT_256 : -1;
+  const int tile = !vec ? -1
+                   : !w4k ? gemm_i8_choose(c, M, N, K, lora ? GT_LORA : g.epi == ANIMA_EPI_STORE ? GT_STORE : GT_RESID)
+                   : few || lora ? -1 : (int)GT_256;
   // the LoRA product in the epilogue: a tile's columns lie in one rank block
   const bool lepi = lora && tile >= 0 && d->lora_cols % gemm_i8_cols(tile) == 0;
   // otherwise the LoRA product is an add term (the split-bf16 kernel, one product per rank block

@@ -492,7 +492,7 @@ int anima_weight_unpack_w4(anima_ctx* ctx, const anima_weight* w4, int8_t* grid)
  *     products of few rows and short or very many columns, and if there is no memory for the
  *     grid.)
  *   ANIMA_W4_IN_GEMM: every workgroup unpacks its B tiles inside the GEMM main loop (no scratch;
- *     with a LoRA the large products still take the grid). */
+ *     with a LoRA, products of more than a few rows still take the grid). */
 #define ANIMA_W4_GRID_SCRATCH 0
 #define ANIMA_W4_IN_GEMM 1
 int anima_set_w4_path(anima_ctx* ctx, int path);

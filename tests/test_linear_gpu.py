@@ -365,12 +365,13 @@ def test_int8_tile_sizes(ctx, M, N, K, kind):
 
 @pytest.mark.parametrize("M,N,K,lora,kernel", [
     (4096, 6144, 128, 0, "gemm.w4a8.256x256"), (2300, 8196, 192, 0, "gemm.w4a8.256x256"),
-    (1000, 2048, 128, 0, "gemm.w4a8.general"), (4096, 6146, 64, 0, "gemm.w4a8.general"),
-    (4100, 4100, 128, 32, "gemm.i8."), (1000, 2048, 128, 32, "gemm.w4a8.general")])
+    (1000, 2048, 128, 0, "gemm.w4a8.256x256"), (33, 2052, 192, 0, "gemm.w4a8.256x256"), (32, 2048, 128, 0, "gemm.w4a8.general"),
+    (4096, 6146, 64, 0, "gemm.w4a8.general"),
+    (4100, 4100, 128, 32, "gemm.i8."), (1000, 2048, 128, 32, "gemm.i8."), (30, 2048, 128, 32, "gemm.w4a8.general")])
 def test_w4_in_gemm_kernels(ctx, w4_path, M, N, K, lora, kernel):
-    """W4 codes decoded inside the GEMM: products with a 256x256 tile for every CU run the 256x256 kernel (whatever tile
-    the same product takes on int8 weights), the rest the general one; with a LoRA the first run on the scratch grid
-    with the term in the epilogue.  Exact sums; bits of the same product on the int8 grid."""
+    """W4 codes decoded inside the GEMM: products of more than 32 rows run the 256x256 kernel (whatever tile the same
+    product takes on int8 weights), the rest the general one; with a LoRA the first run on the scratch grid with the
+    term in the epilogue.  Exact sums; bits of the same product on the int8 grid."""
     case(f"W4 in the GEMM M={M} N={N} K={K} lora={lora}")
     m = amd()
     codes, srel, sw = w4_weight(K, N, K)
