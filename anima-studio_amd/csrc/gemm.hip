@@ -2582,10 +2582,10 @@ static int gemm_i8_cols(int tile) { return tile == GT_256 ? 256 : tile == GT_32x
 // Microseconds of a product on one tile size: base (launch, first loads, the last epilogue) + for each tile per CU
 // step * K / 2048, and round for each one after the first (its epilogue).  Per epilogue: the stored output is much of a
 // short product.  Fitted to 3276 products of M = 1 .. 16384, N = 64 .. 8192, K = 64 .. 8192 (1575 with a LoRA, 900
-// with attention operands): the choice takes 1.1 / 0.4% longer than the best tile in the mean (plain / residual), 0.3%
-// the others.  The constants of one sum per tile, fitted at K >= 2048, took 12 / 8 / 9% at all K (4096 x 4096 x 64: 32x64 tiles 43 us,
+// with attention operands): the choice takes 1.9 / 0.4% longer than the best tile in the mean (plain / residual), 0.2
+// to 0.5% the others.  The constants of one sum per tile, fitted at K >= 2048, took 12 / 8 / 9% at all K (4096 x 4096 x 64: 32x64 tiles 43 us,
 // 256x256 26).  Another tile than 256x256 has to be 4% faster where that one has a tile for every CU (it varies least
-// from run to run), and stored products of K < 512 stay there (bound by their stores: 12288 x 2048 x 128 26 us, 128x128 32).
+// from run to run), and stored products of K <= 128 stay there (bound by their stores: 12288 x 2048 x 128 26 us, 128x128 32).
 static int gemm_i8_choose(anima_ctx* c, int64_t M, int N, int K, int kind) {
   static const struct { int bm, bn; } T[GT_COUNT] = {{256, 256}, {256, 128}, {128, 128}, {64, 128}, {32, 64}};
   static const struct { float base, step, round; } P[5][GT_COUNT] = {
@@ -2593,7 +2593,7 @@ static int gemm_i8_choose(anima_ctx* c, int64_t M, int N, int K, int kind) {
       {{15.6f, 16.3f, 27.8f}, {15.3f, 8.9f, 17.5f}, {6.2f, 7.3f, 6.3f}, {5.9f, 5.6f, 5.3f}, {3.8f, 1.9f, 1.0f}},    // residual, gate
       {{41.5f, 21.0f, 56.2f}, {16.2f, 10.3f, 32.6f}, {12.5f, 7.4f, 12.4f}, {10.0f, 4.9f, 10.9f}, {}},               // LoRA
       {{29.8f, 20.8f, 31.5f}, {16.5f, 13.2f, 15.8f}, {12.1f, 9.4f, 4.9f}, {7.1f, 6.1f, 2.2f}, {}},                  // operands
-      {{39.6f, 37.6f, 44.3f}, {19.8f, 11.3f, 24.6f}, {16.2f, 8.4f, 7.6f}, {7.5f, 5.5f, 4.0f}, {}}};                 // operands + LoRA
+      {{44.8f, 37.6f, 44.3f}, {19.8f, 10.3f, 25.6f}, {13.6f, 8.2f, 7.8f}, {7.5f, 6.1f, 4.0f}, {}}};                 // operands + LoRA
   int best = -1;
   float bt = 0.0f;
   for (int t = 0; t < GT_COUNT; t++) {
@@ -2603,7 +2603,7 @@ static int gemm_i8_choose(anima_ctx* c, int64_t M, int N, int K, int kind) {
     const float rounds = (float)((tiles + c->num_cus - 1) / c->num_cus);
     float us = P[kind][t].base + P[kind][t].step * (float)K / 2048.0f * rounds + P[kind][t].round * (rounds - 1.0f);
     if (t == GT_256 && tiles >= c->num_cus) {
-      if (kind == GT_STORE && K < 512) return GT_256;
+      if (kind == GT_STORE && K <= 128) return GT_256;
       us = us / 1.04f;
     }
     if (best < 0 || us < bt) {

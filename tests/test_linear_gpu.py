@@ -487,7 +487,7 @@ def test_256_tile_kernel_activation_epilogues(ctx, act, epi):
     (3900, 3900, 1024, "i8", "gated", "none", "bias", "gemm.i8.256x256"),
     (3900, 3900, 1024, "i8", "gated", "none", "bias add", "gemm.i8.256x256"),
     (8100, 4060, 1024, "i8", "resid", "silu", "", "gemm.i8.256x256"),
-    (4500, 4100, 192, "i8", "store", "gelu", "bias", "gemm.i8.256x256"),
+    (4500, 4100, 128, "i8", "store", "gelu", "bias", "gemm.i8.256x256"),
     (4500, 4100, 64, "w4", "store", "none", "bias", "gemm.i8.256x256"),
     (3900, 3900, 192, "w4", "resid", "none", "", "gemm.i8.256x256"),
     (3900, 3900, 1024, "i8", "gated", "none", "bias lora48", "gemm.i8.256x256"),
