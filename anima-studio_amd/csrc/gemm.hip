@@ -2676,8 +2676,10 @@ static void s3_lds_launch(anima_ctx* c, const F32WArgs& f, int ks) {
     else if (nch % 2 == 0) S3L(2, 2);
     else S3L(2, 1);
   } else {  // several workgroups per CU: four steps ahead took 5 to 15% longer than two
-    if (nch % 2) S3L(1, 1, true);
-    else if (nch <= 12) S3L(1, 2, true);  // (5420 x 808 x 128 16.5 -> 15.8 us; 1024 x 2304 x 2048 47.6 and 46.7 without)
+    const bool shrt = nch <= 12;
+    if (nch % 2 && shrt) S3L(1, 1, true);
+    else if (nch % 2) S3L(1, 1);
+    else if (shrt) S3L(1, 2, true);  // (5420 x 808 x 128 16.5 -> 15.8 us; 1024 x 2304 x 2048 47.6 and 46.7 without)
     else S3L(1, 2);
   }
 #undef S3L
