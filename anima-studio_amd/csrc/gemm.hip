@@ -4,7 +4,7 @@
 //   gemm_i8   C = epi((qx @ qw^T) * s_x[m] * s_w[n]) with v_mfma_i32_32x32x32_i8 (exact int32
 //             accumulation): gemm_i8_256 and the smaller tiles of gemm_i8_tile, chosen by size, on
 //             int8 weights (W4: on the unpacked grid); gemm_i8_kernel for unaligned rows, rows of
-//             2^23 weights and more, and W4 weights decoded inside a product of up to 32 rows:
+//             2^23 weights and more, and W4 weights decoded inside a product of few rows or few tiles:
 //             block tile 128x128, k-tile 64, 4 waves of 64x64, double-buffered LDS with 80-byte rows
 //             (conflict-free 16-byte fragment reads).
 //             W4: the weight tile is decoded in the loader, nibble -> int8 grid value through a
@@ -2949,6 +2949,9 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
   // of the two kernels that decode W4 codes, the 256x256 one runs its decode beside the matrix cores: shorter for all but
   // few rows (2112 x 6144 x 4864 101 us, gemm_i8_kernel 230; 43 x 2048 x 64 10.2 and 18.8; 1 x 2048 x 2048 30.5 and 23.1)
   const bool few = M <= (K > 4096 ? 64 : 32) || tiles256 > 0x7fffffff;
+  // (of long sums over few tiles gemm_i8_kernel is the shorter: 3077 x 64 x 6720 77.7 us, the 256x256 kernel 86.4; over
+  // 3257 products of K > 4096 the line drawn here takes 0.7% longer than the better of the two in the mean, by rows alone 3.9%)
+  const bool few_tiles = K > 4096 && (int64_t)((N + 127) / 128) * ((M + 127) / 128) <= (K < 8192 ? 32 : 16);
   void* grid8 = nullptr;
   bool w4k = w4;  // the GEMM unpacks W4 codes itself
   // (the LoRA epilogue of a tile runs on the int8 grid: the in-GEMM unpack leaves it no registers, and an add term
@@ -2966,7 +2969,7 @@ int linear_launch(anima_ctx* c, const anima_linear_desc* d, int64_t s3_plane) {
   }
   const int tile = !vec ? -1
                    : !w4k ? gemm_i8_choose(c, M, N, K, lora ? GT_LORA : g.epi == ANIMA_EPI_STORE ? GT_STORE : GT_RESID)
-                   : few || lora ? -1 : (int)GT_256;
+                   : few || few_tiles || lora ? -1 : (int)GT_256;
   // the LoRA product in the epilogue: a tile's columns lie in one rank block
   const bool lepi = lora && tile >= 0 && d->lora_cols % gemm_i8_cols(tile) == 0;
   // otherwise the LoRA product is an add term (the split-bf16 kernel, one product per rank block

@@ -366,11 +366,14 @@ def test_int8_tile_sizes(ctx, M, N, K, kind):
 @pytest.mark.parametrize("M,N,K,lora,kernel", [
     (4096, 6144, 128, 0, "gemm.w4a8.256x256"), (2300, 8196, 192, 0, "gemm.w4a8.256x256"),
     (1000, 2048, 128, 0, "gemm.w4a8.256x256"), (33, 2052, 192, 0, "gemm.w4a8.256x256"), (32, 2048, 128, 0, "gemm.w4a8.general"),
+    (129, 2052, 4160, 0, "gemm.w4a8.256x256"), (129, 2048, 4160, 0, "gemm.w4a8.general"),
+    (257, 1024, 8192, 0, "gemm.w4a8.256x256"), (256, 1024, 8192, 0, "gemm.w4a8.general"),
     (4096, 6146, 64, 0, "gemm.w4a8.general"),
     (4100, 4100, 128, 32, "gemm.i8."), (1000, 2048, 128, 32, "gemm.i8."), (30, 2048, 128, 32, "gemm.w4a8.general")])
 def test_w4_in_gemm_kernels(ctx, w4_path, M, N, K, lora, kernel):
-    """W4 codes decoded inside the GEMM: products of more than 32 rows run the 256x256 kernel (whatever tile the same
-    product takes on int8 weights), the rest the general one; with a LoRA the first run on the scratch grid with the
+    """W4 codes decoded inside the GEMM: products of more than 32 rows (64 at K > 4096, and there more than 32, from
+    K = 8192 16, tiles of 128x128) run the 256x256 kernel (whatever tile the same product takes on int8 weights), the rest
+    the general one; with a LoRA the first run on the scratch grid with the
     term in the epilogue.  Exact sums; bits of the same product on the int8 grid."""
     case(f"W4 in the GEMM M={M} N={N} K={K} lora={lora}")
     m = amd()
@@ -392,7 +395,7 @@ def test_w4_in_gemm_kernels(ctx, w4_path, M, N, K, lora, kernel):
     names = ran(ctx, lambda: ctx.linear(W, M, out, xq=dq, xs=ds, epilogue=m.EPI_RESID, acc_out=acc, **kw))
     assert any(n.startswith(kernel) for n in names), names
     assert ("gemm.f32s3" in names) == (lora > 0 and kernel == "gemm.w4a8.general"), names  # the LoRA term as an add term
-    assert np.array_equal(acc.numpy(), (q.astype(np.float32) @ grid.astype(np.float32).T).astype(np.int32))  # |sums| < 2^24
+    assert np.array_equal(acc.numpy(), (q.astype(np.float64) @ grid.astype(np.float64).T).astype(np.int32))  # exact: |sums| < 2^53
     ctx.linear(W8, M, out8, xq=dq, xs=ds, epilogue=m.EPI_RESID, **kw)
     if lora:
         assert report("against the int8 grid", out.numpy(), out8.numpy())[0] <= 2e-6
