@@ -1384,14 +1384,21 @@ static int attention_check(anima_ctx* c, const anima_attn_desc* d, int (&kv_len)
 // Key groups of the fp32 kernel, by the measured time of both forms (us; n blocks of 64 keys): 128-query
 // workgroups run two to a CU in 16.4 n + 16, a single one in 9 n + 12; a 64-query workgroup with two key groups takes
 // 10.4 ceil(n / 2) + 14, one to a CU.  Under a causal mask of several blocks the second form balances better
-// (4096 tokens, 16 heads: 860 us, the first 1056).
+// (4096 tokens, 16 heads: 860 us, the first 1056) unless at least a third of the queries see all keys: there its time is
+// that of the mean blocks of a query, the last round half full (2 x 2641 queries, 20 heads of 128, 317 keys: 291 us, the
+// first form 197; 4116 queries, 4 heads of 64, 1372 keys: 141 and 203).
 static int fp32_key_groups(int num_cus, const anima_attn_desc* d) {
   const int64_t bh = (int64_t)d->B * d->H, n = d->causal ? std::min((d->Lk + BK - 1) / BK, (d->Lq + BK - 1) / BK) : (d->Lk + BK - 1) / BK;
-  if (d->causal && n > 1) return 2;
+  const bool masked = d->causal && n > 1;
+  if (masked && 2 * (int64_t)d->Lq < 3 * (int64_t)d->Lk) return 2;
   const int64_t w1 = (bh * ((d->Lq + BQ32<1> - 1) / BQ32<1>) + num_cus - 1) / num_cus,
                 w2 = (bh * ((d->Lq + BQ32<2> - 1) / BQ32<2>) + num_cus - 1) / num_cus;
   const double t1 = (double)(w1 / 2) * (16.4 * n + 16) + (double)(w1 % 2) * (9.0 * n + 12),
                t2 = (double)w2 * (10.4 * ((n + 1) / 2) + 14);
+  if (masked) {
+    const double seen = 1.0 - 0.5 * d->Lk / d->Lq, rounds = (double)(bh * ((d->Lq + BQ32<2> - 1) / BQ32<2>)) / num_cus + 0.5;
+    return t1 <= std::min(t2, std::max(rounds, 1.0) * (10.4 * ((n + 1) / 2) * seen + 14)) ? 1 : 2;
+  }
   return t1 <= t2 ? 1 : 2;
 }
 

@@ -366,11 +366,13 @@ def test_head_dim_64_flash_path(ctx, precision):
     (2, 6, 400, 4, 2, 1, [400, 3], "attn.flash_fp32"), (1, 64, 300, 2, 1, 1, None, "attn.flash_fp32"),
     (4, 300, 200, 16, 2, 0, [200, 64, 1, 130], "attn.flash_fp32"), (2, 1300, 512, 8, 1, 0, [449, 512], "attn.flash_fp32"),
     (1, 129, 200, 2, 1, 0, None, "attn.flash_fp32_2g"), (2, 65, 320, 4, 2, 0, [320, 63], "attn.flash_fp32_2g"),
-    (1, 192, 192, 2, 1, 1, None, "attn.flash_fp32_2g"), (3, 130, 77, 2, 1, 1, [77, 70, 5], "attn.flash_fp32_2g")])
+    (1, 192, 192, 2, 1, 1, None, "attn.flash_fp32_2g"), (3, 130, 77, 2, 1, 1, [77, 70, 5], "attn.flash_fp32_2g"),
+    (4, 1000, 128, 16, 2, 1, [128, 77, 1, 100], "attn.flash_fp32"), (2, 1321, 317, 20, 4, 1, None, "attn.flash_fp32"),
+    (1, 640, 200, 20, 1, 1, None, "attn.flash_fp32_2g")])
 def test_fp32_forms(ctx, B, Lq, Lk, H, group, causal, kv_len, form):
     """Both forms of the fp32 kernel (128-query workgroups on all keys; 64-query ones with two key groups) where the
     rule takes them, with remainders in queries and keys, masks and grouped heads, against float64; few keys under
-    many queries run the first form (the second leaves half of each workgroup idle there)."""
+    many queries run the first form (the second leaves half of each workgroup idle there), also behind a causal mask."""
     case(f"fp32 attention {form} B={B} Lq={Lq} Lk={Lk} H={H} causal={causal}")
     m = amd()
     D, Hk = HD, H // group
